@@ -30,6 +30,7 @@ SOURCES = (
     "attention_fwd.hip",
     "attention_scaled.hip",
     "linear_gelu.hip",
+    "linear_tiles.hip",
     "gelu.hip",
     "linear_norm.hip",
     "mlp_norm.hip",
@@ -47,12 +48,14 @@ HIPCC_FLAGS = (
     "-target-feature",
     "-Xclang",
     "-packed-fp32-ops",
-    # MFMA accumulators in ordinary VGPRs (gfx950 reads/writes C and D from the
-    # unified file); avoids v_accvgpr read/write traffic around VALU updates.
-    "-mllvm",
-    "-amdgpu-mfma-vgpr-form",
 )
 
+# MFMA accumulators in ordinary VGPRs (gfx950 reads/writes C and D from the
+# unified file); avoids v_accvgpr read/write traffic around VALU updates.
+VGPR_FORM = ("-mllvm", "-amdgpu-mfma-vgpr-form")
+# linear_tiles.hip keeps the default: its 256 x 256 tile holds 256 accumulators
+# per lane at one wave per SIMD, which only fit beside the operands as AGPRs.
+AGPR_SOURCES = ("linear_tiles.hip",)
 
 # Per-source additions.  attention_fwd.hip (the plain attention path and the
 # other attention kernels): LLVM's max-memory-clause machine scheduler
@@ -138,7 +141,8 @@ def build(verbose: bool = False) -> Path:
 
     def compile_one(source: str) -> Path:
         obj = BUILD_DIR / (Path(source).stem + ".o")
-        _run([hipcc, *HIPCC_FLAGS, *SOURCE_FLAGS.get(source, ()), "-c", str(CSRC / source), "-o", str(obj)], verbose)
+        form = () if source in AGPR_SOURCES else VGPR_FORM
+        _run([hipcc, *HIPCC_FLAGS, *form, *SOURCE_FLAGS.get(source, ()), "-c", str(CSRC / source), "-o", str(obj)], verbose)
         return obj
 
     with concurrent.futures.ThreadPoolExecutor(max_workers=len(SOURCES)) as pool:

@@ -33,10 +33,10 @@ __global__ __launch_bounds__(512) void gelu_kernel(const T* x, T* y, int64_t n) 
     if (idx + 8 <= n) {
       V8 v = __builtin_bit_cast(V8, raw[c]);
 #pragma unroll
-      for (int e = 0; e < 8; ++e) v[e] = from_f32<T>(gelu_exact(to_f32(v[e])));
+      for (int e = 0; e < 8; ++e) v[e] = from_f32<T>(fp32_result<T>(gelu_exact(to_f32(v[e]))));
       store16(y + idx, __builtin_bit_cast(u32x4, v));
     } else if (idx < n) {  // the ragged end: fewer than 8 elements left
-      for (int64_t e = idx; e < n; ++e) y[e] = from_f32<T>(gelu_exact(to_f32(x[e])));
+      for (int64_t e = idx; e < n; ++e) y[e] = from_f32<T>(fp32_result<T>(gelu_exact(to_f32(x[e]))));
     }
   }
 }

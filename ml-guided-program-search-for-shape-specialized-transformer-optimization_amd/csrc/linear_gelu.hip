@@ -7,20 +7,23 @@
 // fp32 and one rounding to the output dtype.  With the activation switched off
 // the same kernel is a plain Linear (bias optional).
 //
-// MI355X formulation:
-//  * 256 x 256 output tile per workgroup of 8 wavefronts (2 x 4), each wave
+// MI355X formulation: the direct-to-LDS tile kernels of linear_tiles.hip,
+// chosen by size.  The kernel in this file stages its operands through
+// registers and remains for the two cases the others do not take: a LayerNorm
+// applied to x on its way into LDS, and x rows further apart than the
+// direct loads' 32-bit offsets reach.  It is
+//  * a 256 x 256 output tile per workgroup of 8 wavefronts (2 x 4), each wave
 //    owning 128 rows x 64 columns; K advances 64 at a time through a
 //    double-buffered LDS stage (rows padded by 16 bytes, conflict-free 16-byte
-//    operand reads) with one barrier per K step.
-//  * The product is computed transposed, Y^T = W X^T, with
+//    operand reads) with one barrier per K step;
+//  * the product computed transposed, Y^T = W X^T, with
 //    v_mfma_f32_32x32x16_{bf16,f16}: both operands are 16-byte row chunks of
 //    the row-major x and W tiles, and every lane's accumulator column is one
 //    output row holding runs of 4 consecutive output columns, so the epilogue
 //    packs them into 8-byte LDS writes and the tile leaves through LDS as
-//    fully coalesced 16-byte stores.
-//  * Workgroup ids are remapped so that each XCD (ids are dealt round-robin
-//    over the 8 XCDs) works on a contiguous run of tiles: the x rows of a
-//    run's tiles are shared in that XCD's L2.
+//    fully coalesced 16-byte stores;
+//  * workgroup ids remapped so that each XCD (ids are dealt round-robin
+//    over the 8 XCDs) works on a contiguous run of tiles.
 //
 // The same GEMM with a head-major epilogue is the packed QKV projection of the
 // reference's native-layout path (solution/kernels/projection/
@@ -46,7 +49,7 @@
 
 #include <cmath>
 
-#include "sah_common.hpp"
+#include "linear_tiles.hpp"
 
 namespace sah {
 namespace {
@@ -58,37 +61,6 @@ constexpr int kWaves = 8;
 constexpr int kThreads = kWaves * 64;
 constexpr int kRow = kBK + 8;         // LDS operand row (elements), 16-byte pad
 constexpr int kOutRow = kBN + 8;      // LDS output staging row (elements)
-
-// Epilogues: row-major y (optionally through exact GELU), or the head-major
-// Q / K / V scatter.
-constexpr int kEpiRows = 0;
-constexpr int kEpiRowsGelu = 1;
-constexpr int kEpiHeads = 2;
-
-struct LinearParams {
-  const void* x;     // [rows][K], row stride x_ld
-  const void* w;     // [N][K], contiguous
-  const void* bias;  // [N] or null, same dtype as x
-  void* y;           // [rows][N], row stride y_ld (row-major epilogues)
-  int64_t rows, x_ld, y_ld;
-  int n, k;
-  int tiles_n, num_tiles;
-  // Head-major epilogue: output columns [0, D) -> q, [D, 2D) -> k,
-  // [2D, 3D) -> v, column c of a block -> head c / head_dim, element
-  // c % head_dim; row r -> token (r / seq_len, r % seq_len).
-  void* q;
-  void* kk;
-  void* v;
-  int64_t v_ld;      // seq stride of a seq-contiguous value
-  int seq_len, heads, head_dim, d_model;
-  int v_seq_major;   // value as [B][H][head_dim][v_ld] instead of [B][H][S][head_dim]
-  int seq_aligned;   // seq_len % 8 == 0: 8-token runs never cross a sequence
-  // LayerNorm on the x rows: weight / bias [K] in the x dtype and each
-  // row's (mean, 1/std).
-  const void* ln_w;
-  const void* ln_b;
-  const float2* ln_stats;
-};
 
 // Row statistics of G rows of K = ITERS * 512 elements by one wavefront,
 // exactly as the fused norm kernel forms them: lane l holds elements
@@ -173,25 +145,15 @@ int row_stats(const void* x, int64_t x_ld, int64_t rows, int64_t k, float eps, f
   }
 }
 
-__device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ f32x16 mfma32(f16x8 a, f16x8 b, f32x16 c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0);
-}
-
 template <typename T, int EPI, bool LN = false>
 __global__ __launch_bounds__(kThreads) void linear_kernel(LinearParams p) {
   typedef typename Vec8<T>::type V8;
-  typedef typename Vec8<T>::half_type V4;
-  constexpr bool GELU = EPI == kEpiRowsGelu;
 
   // Two operand stages of x and W rows; after the K loop the same bytes hold
   // the output tile.
   __shared__ __attribute__((aligned(16))) unsigned char smem[2 * 2 * kBM * kRow * sizeof(T)];
   T(*x_lds)[kBM][kRow] = reinterpret_cast<T(*)[kBM][kRow]>(smem);
   T(*w_lds)[kBN][kRow] = reinterpret_cast<T(*)[kBN][kRow]>(smem + 2 * kBM * kRow * sizeof(T));
-  T(*y_lds)[kOutRow] = reinterpret_cast<T(*)[kOutRow]>(smem);
   static_assert(kBM * kOutRow * sizeof(T) <= sizeof(smem), "output staging must fit");
 
   const int tid = threadIdx.x;
@@ -318,111 +280,17 @@ __global__ __launch_bounds__(kThreads) void linear_kernel(LinearParams p) {
     __syncthreads();
   }
 
-  // ---- epilogue: bias, activation, one rounding; stage the tile in LDS.
-  // Accumulator register r of acc[i][j] holds output column
-  // 32 i + 8 (r / 4) + 4 half + r % 4 (within the wave's slab) of row 32 j + l32.
-  const T* bg = static_cast<const T*>(p.bias);
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int n_l = wave_n * 64 + 32 * i + 8 * g + 4 * half;
-      float bv[4] = {0.0f, 0.0f, 0.0f, 0.0f};
-      if (bg != nullptr) {
-        const V4 raw = *reinterpret_cast<const V4*>(bg + n0 + n_l);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) bv[q] = to_f32(raw[q]);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        V4 out;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          float v = acc[i][j][4 * g + q] + bv[q];
-          if (GELU) v = gelu_exact(v);
-          out[q] = from_f32<T>(v);
-        }
-        *reinterpret_cast<V4*>(&y_lds[wave_m * 128 + 32 * j + l32][n_l]) = out;
-      }
-    }
-  }
-  __syncthreads();
-
-  constexpr int kChunks = (kBM * kBN / 8) / kThreads;  // 16-byte chunks per thread
-  if constexpr (EPI != kEpiHeads) {
-    // ---- coalesced 16-byte stores of the valid rows.
-    T* yg = static_cast<T*>(p.y);
-#pragma unroll
-    for (int s2 = 0; s2 < kChunks; ++s2) {
-      const int c = tid + kThreads * s2;
-      const int row = c >> 5;          // 32 chunks of 8 elements per row
-      const int col = (c & 31) * 8;
-      const int64_t m = m0 + row;
-      if (m < p.rows) store16(yg + m * p.y_ld + n0 + col, *reinterpret_cast<const u32x4*>(&y_lds[row][col]));
-    }
-  } else {
-    // ---- head-major scatter.  d_model is a multiple of kBN, so the whole
-    // tile belongs to one of q / k / v.  Token indices fit in 32 bits (the
-    // host checks rows < 2^31).
-    const int which = n0 / p.d_model;
-    const int c0 = n0 - which * p.d_model;
-    T* dst = static_cast<T*>(which == 0 ? p.q : which == 1 ? p.kk : p.v);
-    const unsigned seq = (unsigned)p.seq_len;
-    const int hd = p.head_dim;
-    if (which != 2 || !p.v_seq_major) {
-      // [B][H][S][hd]: a 16-byte chunk is 8 consecutive elements of one head
-      // (head_dim is a multiple of 8).
-#pragma unroll 4
-      for (int s2 = 0; s2 < kChunks; ++s2) {
-        const int c = tid + kThreads * s2;
-        const int row = c >> 5;
-        const int col = (c & 31) * 8;
-        const int64_t m = m0 + row;
-        if (m >= p.rows) continue;
-        const unsigned b = (unsigned)m / seq;
-        const unsigned s = (unsigned)m - b * seq;
-        const int within = c0 + col;
-        const int head = within / hd;
-        const int e = within - head * hd;
-        T* out = dst + (((int64_t)b * p.heads + head) * (int64_t)seq + s) * hd + e;
-        store16(out, *reinterpret_cast<const u32x4*>(&y_lds[row][col]));
-      }
-    } else {
-      // [B][H][hd][v_ld]: a 16-byte chunk is 8 consecutive tokens of one
-      // column, read down an LDS column (consecutive lanes take consecutive
-      // columns: conflict-free).
-#pragma unroll 4
-      for (int s2 = 0; s2 < kChunks; ++s2) {
-        const int c = tid + kThreads * s2;
-        const int col = c & (kBN - 1);
-        const int row0 = (c >> 8) * 8;
-        const int64_t m = m0 + row0;
-        if (m >= p.rows) continue;
-        const int within = c0 + col;
-        const int head = within / hd;
-        const int e = within - head * hd;
-        if (p.seq_aligned && m + 8 <= p.rows) {
-          const unsigned b = (unsigned)m / seq;
-          const unsigned s = (unsigned)m - b * seq;
-          V8 run;
-#pragma unroll
-          for (int t = 0; t < 8; ++t) run[t] = y_lds[row0 + t][col];
-          T* out = dst + (((int64_t)b * p.heads + head) * hd + e) * p.v_ld + s;
-          store16(out, __builtin_bit_cast(u32x4, run));
-        } else {
-          for (int t = 0; t < 8 && m + t < p.rows; ++t) {
-            const unsigned b = (unsigned)(m + t) / seq;
-            const unsigned s = (unsigned)(m + t) - b * seq;
-            dst[(((int64_t)b * p.heads + head) * hd + e) * p.v_ld + s] = y_lds[row0 + t][col];
-          }
-        }
-      }
-    }
-  }
+  store_tile<T, EPI, kBM, kBN, 2, 4>(p, smem, m0, n0, acc);
 }
 
 template <typename T, int EPI, bool LN = false>
 int launch_linear(const LinearParams& prm, hipStream_t stream) {
+  if constexpr (!LN) {
+    if (prm.x_ld <= kMaxTileStride) {
+      if (EPI == kEpiHeads && prm.v_seq_major) return launch_linear_tiles<T, kEpiHeadsSeqValue>(prm, stream);
+      return launch_linear_tiles<T, EPI>(prm, stream);
+    }
+  }
   hipLaunchKernelGGL((linear_kernel<T, EPI, LN>), dim3(prm.num_tiles), dim3(kThreads), 0, stream, prm);
   return check_hip(hipGetLastError(), "linear kernel launch");
 }

@@ -1,0 +1,387 @@
+// Direct-to-LDS tile kernels of the projections (gfx950): Linear, Linear +
+// exact GELU, and the packed QKV projection with its head-major stores.
+//
+// What bounds them: the matrix cores, under the power limit.  The
+// register-staged 8-wave kernel of linear_gelu.hip ran its MFMAs 55% of the
+// time (one __syncthreads per K step with every load behind it, 192 KB of
+// operand reads per step and CU, scalar bias loads in the epilogue) and
+// left most CUs idle for few rows.  Here a 256 x 256 tile is held by four
+// waves, one per SIMD, 128 x 128 each: a third fewer LDS reads per MFMA, and
+// one wave's instruction stream keeps its matrix core busy (2180 cycles per
+// K step against 2048 of MFMAs at 20002 x 1024 -> 3072; 72% of all cycles at
+// 65536 x 2048 -> 8192, where the chip then runs at 1.5 GHz).  Measured with
+// the same inputs on one box, before -> after:
+//   65536 x 2048 -> 8192    2567 -> 1710 us (1286 TFLOP/s), GELU 2786 -> 1960 us
+//   20002 x 1024 -> 3072     154 ->  118 us, GELU 179 -> 157 us
+//   777 x 1024 -> 4096        36 ->   13 us, GELU  44 ->  15 us
+// Tried and slower at 65536 x 2048 -> 8192: two groups of four waves half a
+// step apart on 128 x 64 wave tiles (1983 us); stores of a tile spread over
+// the next tile's main loop from registers (1790 us: 32-byte segments and
+// spills); loads of the next tile between the epilogue's blocks (1830 us,
+// spills; kept for the 128 x 256 tile, which has the registers).
+
+#include "linear_tiles.hpp"
+
+namespace sah {
+namespace {
+
+// The bias of a wave's NI * 32 columns, two per lane (one register): dword d
+// is columns 2 d and 2 d + 1.
+template <typename T, int NI>
+struct WaveBias {
+  uint32_t pair;
+  __device__ __forceinline__ void load(const T* bias, int n_wave) {
+    const int lane = threadIdx.x & 63;
+    pair = 0;
+    if (bias != nullptr && lane < NI * 16) pair = *reinterpret_cast<const uint32_t*>(bias + n_wave + 2 * lane);
+  }
+  // Columns 32 i + 8 g + 4 half .. + 3, as accumulator registers 4 g .. 4 g + 3
+  // of acc[i][j] hold them.
+  __device__ __forceinline__ void get(int i, int g, float (&out)[4]) const {
+    typedef typename Vec8<T>::half_type V4;
+    const int half = (threadIdx.x & 63) >> 5;
+    const int source = (16 * i + 4 * g + 2 * half) * 4;
+    u32x2 raw;
+    raw[0] = (uint32_t)__builtin_amdgcn_ds_bpermute(source, (int)pair);
+    raw[1] = (uint32_t)__builtin_amdgcn_ds_bpermute(source + 4, (int)pair);
+    const V4 v = __builtin_bit_cast(V4, raw);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) out[q] = to_f32(v[q]);
+  }
+};
+
+// row / seq_len and its remainder, exact for rows below 2^31
+// (LinearParams::seq_magic; seq_len 1 has magic 0).
+__device__ __forceinline__ void seq_div(const LinearParams& p, uint32_t row, uint32_t& b, uint32_t& s) {
+  b = p.seq_magic == 0 ? row : __umulhi(row, p.seq_magic) >> p.seq_shift;
+  s = row - b * (uint32_t)p.seq_len;
+}
+
+// The epilogue of one wave's NJ x NI blocks: bias, activation, one rounding.
+// 32 rows at a time pass through the wave's own LDS area (32 rows of NI * 64
+// bytes, 16-byte chunk c of row r in slot c ^ f(r): conflict-free both ways)
+// and leave as 16-byte stores of whole NI * 64 byte row segments, so the waves
+// need no barrier and the stages stay free for the next tile's loads.
+// (Stored straight from the accumulator layout, 32-byte segments, the 65536 x
+// 2048 -> 8192 Linear ran 5% slower.)  m_wave, n_wave: the wave's first row
+// and column.  With every row valid the wave issues exactly NJ * NI * 2
+// stores (seq-contiguous values apart), the last two blocks' after
+// prefetch(NJ - 1).  prefetch(j) runs before the arithmetic of block j.
+template <typename T, int EPI, int NI, int NJ, typename F>
+__device__ __forceinline__ void store_wave(const LinearParams& p, unsigned char* area, int64_t m_wave,
+                                           int n_wave, const WaveBias<T, NI>& bias,
+                                           const f32x16 (&acc)[NI][NJ], const F& prefetch) {
+  typedef typename Vec8<T>::type V8;
+  typedef typename Vec8<T>::half_type V4;
+  constexpr bool kHeads = EPI == kEpiHeads || EPI == kEpiHeadsSeqValue;
+  constexpr int CPR = NI * 4;         // 16-byte chunks per row
+  constexpr int ROWS_PER = 64 / CPR;  // rows per store instruction
+  int lane = threadIdx.x & 63;
+  asm volatile("" : "+v"(lane));  // addresses formed here, not kept over the main loop
+  const int l32 = lane & 31;
+  const int half = lane >> 5;
+  auto slot = [](int row, int chunk) { return chunk ^ (CPR == 16 ? row & 15 : (row >> 1) & (CPR - 1)); };
+
+  const int chunk = lane % CPR;
+  const int col = n_wave + chunk * 8;
+  // head-major: the wave's columns lie in one of q / k / v (d_model is a
+  // multiple of the tile width), a chunk in one head
+  T* dst = nullptr;
+  int head = 0, e = 0;
+  const bool v_seq = EPI == kEpiHeadsSeqValue && n_wave >= 2 * p.d_model;
+  if constexpr (kHeads) {
+    const int which = n_wave / p.d_model;
+    dst = static_cast<T*>(which == 0 ? p.q : which == 1 ? p.kk : p.v);
+    const int within = col - which * p.d_model;
+    head = within / p.head_dim;
+    e = within - head * p.head_dim;
+  }
+
+  float bv[NI][4][4];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int g = 0; g < 4; ++g) bias.get(i, g, bv[i][g]);
+
+  // Block j: compute, write to the area, read back row segments; the reads'
+  // latency passes under the next block's first arithmetic, then they are
+  // stored (LDS keeps a wave's reads before its later writes).
+  constexpr int NS = 32 / ROWS_PER;  // stores per block
+  u32x4 segment[NS];
+  auto store_segments = [&](int j) {
+#pragma unroll
+    for (int r = 0; r < NS; ++r) {
+      const int64_t m = m_wave + 32 * j + r * ROWS_PER + lane / CPR;
+      if (kHeads) __builtin_amdgcn_sched_barrier(0);
+      if (m >= p.rows) continue;
+      if constexpr (kHeads) {
+        uint32_t b, s;
+        seq_div(p, (uint32_t)m, b, s);
+        store16(dst + (((int64_t)b * p.heads + head) * (int64_t)p.seq_len + s) * p.head_dim + e, segment[r]);
+      } else {
+        store16(static_cast<T*>(p.y) + m * p.y_ld + col, segment[r]);
+      }
+    }
+  };
+#pragma unroll
+  for (int j = 0; j < NJ; ++j) {
+    prefetch(j);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        V4 out;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          float v = acc[i][j][4 * g + q] + bv[i][g][q];
+          if (EPI == kEpiRowsGelu) v = fp32_result<T>(gelu_exact(v));
+          out[q] = from_f32<T>(v);
+        }
+        *reinterpret_cast<V4*>(area + l32 * (CPR * 16) + slot(l32, 4 * i + g) * 16 + half * 8) = out;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if (i == 0 && j > 0 && !v_seq) store_segments(j - 1);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
+    if (EPI == kEpiHeadsSeqValue && v_seq) {
+      // [B][H][hd][v_ld]: 8 consecutive tokens of one column per 16 bytes
+#pragma unroll 1
+      for (int c = lane; c < 4 * CPR * 8; c += 64) {
+        const int vcol = c % (CPR * 8);
+        const int row0 = c / (CPR * 8) * 8;
+        const int64_t m = m_wave + 32 * j + row0;
+        if (m >= p.rows) continue;
+        const int within = n_wave + vcol - 2 * p.d_model;
+        const int vh = within / p.head_dim;
+        const int ve = within - vh * p.head_dim;
+        V8 run;
+#pragma unroll
+        for (int t = 0; t < 8; ++t)
+          run[t] = *reinterpret_cast<const T*>(area + (row0 + t) * (CPR * 16) + slot(row0 + t, vcol >> 3) * 16 + (vcol & 7) * 2);
+        uint32_t b, s;
+        seq_div(p, (uint32_t)m, b, s);
+        if (p.seq_aligned && m + 8 <= p.rows) {
+          store16(dst + (((int64_t)b * p.heads + vh) * p.head_dim + ve) * p.v_ld + s, __builtin_bit_cast(u32x4, run));
+        } else {
+#pragma unroll
+          for (int t = 0; t < 8; ++t) {
+            if (m + t >= p.rows) break;
+            seq_div(p, (uint32_t)(m + t), b, s);
+            dst[(((int64_t)b * p.heads + vh) * p.head_dim + ve) * p.v_ld + s] = run[t];
+          }
+        }
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < NS; ++r) {
+        const int row = r * ROWS_PER + lane / CPR;
+        segment[r] = *reinterpret_cast<const u32x4*>(area + row * (CPR * 16) + slot(row, chunk) * 16);
+      }
+    }
+    __builtin_amdgcn_wave_barrier();
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (!v_seq) store_segments(NJ - 1);
+}
+
+// Tile `logical` of the launch: groups of group_m row tiles walked column by
+// column, so the tiles an XCD works on at a time share both x rows and w rows
+// in its L2.
+__device__ __forceinline__ void tile_at(const LinearParams& p, int logical, int& tile_m, int& tile_n) {
+  const int group_tiles = p.group_m * p.tiles_n;
+  const int group = logical / group_tiles;
+  const int first = group * p.group_m;
+  const int height = p.tiles_m - first < p.group_m ? p.tiles_m - first : p.group_m;
+  const int in_group = logical - group * group_tiles;
+  tile_n = in_group / height;
+  tile_m = first + in_group - tile_n * height;
+}
+
+template <int NI, int NJ>
+__device__ __forceinline__ void clear(f32x16 (&acc)[NI][NJ]) {
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < NJ; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
+}
+
+// One tile per workgroup, the four-stage ring.
+template <typename T, int EPI, int TM, int TN, int WM, int WN>
+__global__ __launch_bounds__(WM * WN * 64) void linear_ring_kernel(LinearParams p) {
+  typedef GemmTile<T, TM, TN, WM, WN> Tile;
+  constexpr uint32_t kStageBytes = Tile::RING * (Tile::XSTAGE + Tile::WSTAGE);
+  constexpr uint32_t kAreaBytes = 32 * Tile::COLS * sizeof(T);
+  __shared__ __attribute__((aligned(16))) unsigned char smem[kStageBytes + Tile::WAVES * kAreaBytes];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+
+  // contiguous runs of tiles per XCD (ids are dealt round-robin over the 8)
+  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+  const int per = p.num_tiles >> 3, rem = p.num_tiles & 7;
+  int tile_m, tile_n;
+  tile_at(p, xcd * per + (xcd < rem ? xcd : rem) + local, tile_m, tile_n);
+  const int64_t m0 = (int64_t)tile_m * TM;
+  const int n0 = tile_n * TN;
+  Tile tile;
+  tile.init(smem, Tile::RING * Tile::XSTAGE);
+  const int64_t left = p.rows - m0;
+  tile.operands(static_cast<const T*>(p.x) + m0 * p.x_ld, p.x_ld, left < TM ? (int)left : TM,
+                static_cast<const T*>(p.w) + (int64_t)n0 * p.k, p.k);
+  const int n_wave = n0 + wave % WN * Tile::COLS;
+  WaveBias<T, Tile::NI> bias;
+  bias.load(static_cast<const T*>(p.bias), n_wave);
+  f32x16 acc[Tile::NI][Tile::NJ];
+  clear(acc);
+  tile.ring(smem, p.k / kTileK, acc);
+  store_wave<T, EPI>(p, smem + kStageBytes + wave * kAreaBytes, m0 + wave / WN * Tile::ROWS, n_wave, bias,
+                     acc, [](int) {});
+}
+
+// Persistent workgroups of four waves, one per CU, each walking tiles of its
+// XCD's contiguous run.  A tile's output is finished in registers while the
+// next tile's first loads are under way, and stored between the MFMAs of the
+// next tile's first steps: at the end of a tile all CUs would otherwise wait
+// for 32 MB of stores at once.
+template <typename T, int EPI, int TM, int TN>
+__global__ __launch_bounds__(256, 1) void linear_deep_kernel(LinearParams p) {
+  typedef GemmTile<T, TM, TN, 2, 2> Tile;
+  constexpr uint32_t kStageBytes = 2 * (Tile::XSTAGE + Tile::WSTAGE);
+  constexpr uint32_t kAreaBytes = 32 * Tile::COLS * sizeof(T);
+  // Stores of a wave's full epilogue, all issued after the last of the next
+  // tile's loads.
+  constexpr int kBehind = 2 * Tile::NI * Tile::NJ;
+  __shared__ __attribute__((aligned(16))) unsigned char smem[kStageBytes + 4 * kAreaBytes];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+
+  const int xcd = blockIdx.x & 7, local = blockIdx.x >> 3;
+  const int per = p.num_tiles >> 3, rem = p.num_tiles & 7;
+  const int run = xcd * per + (xcd < rem ? xcd : rem);  // the XCD's first tile
+  const int end = run + per + (xcd < rem ? 1 : 0);
+  const int stride = (gridDim.x + 7 - xcd) >> 3;        // workgroups of this XCD
+  const int steps = p.k / kTileK;
+
+  Tile tile;
+  tile.init(smem, 2 * Tile::XSTAGE);
+  int64_t m0 = 0;
+  int n0 = 0;
+  auto begin = [&](int logical) {
+    int tile_m, tile_n;
+    tile_at(p, logical, tile_m, tile_n);
+    m0 = (int64_t)tile_m * TM;
+    n0 = tile_n * TN;
+    const int64_t left = p.rows - m0;
+    tile.operands(static_cast<const T*>(p.x) + m0 * p.x_ld, p.x_ld, left < TM ? (int)left : TM,
+                  static_cast<const T*>(p.w) + (int64_t)n0 * p.k, p.k);
+  };
+  int logical = run + local;
+  if (logical >= end) return;
+  begin(logical);
+  tile.template deep_prefetch<0, 1>(steps);
+  // The number of stores issued after the loads of step 0 is known (kBehind
+  // or more), so those loads can be waited for without waiting for the stores.
+  bool stores_behind = false;
+  while (true) {
+    if (stores_behind)
+      wait_loads<kBehind>();
+    else
+      wait_loads<0>();
+    tile_barrier();
+    const int64_t m_wave = m0 + wave / 2 * Tile::ROWS;
+    const int n_wave = n0 + wave % 2 * Tile::COLS;
+    const bool full = m0 + TM <= p.rows && EPI != kEpiHeadsSeqValue;
+    WaveBias<T, Tile::NI> bias;
+    bias.load(static_cast<const T*>(p.bias), n_wave);
+    f32x16 acc[Tile::NI][Tile::NJ];
+    clear(acc);
+    tile.deep(smem, steps, acc);
+    logical += stride;
+    const bool more = logical < end;
+    if (more) begin(logical);
+    // TN 256 x TM 256 has no registers to spare for loads between the blocks
+    if (Tile::NJ > 2 && more) tile.template deep_prefetch<0, 1>(steps);
+    store_wave<T, EPI>(p, smem + kStageBytes + wave * kAreaBytes, m_wave, n_wave, bias, acc, [&](int j) {
+      if (Tile::NJ > 2 || !more) return;
+      if (j == 0) tile.template deep_prefetch<0, 2>(steps);
+      if (j == 1) tile.template deep_prefetch<1, 2>(steps);
+    });
+    if (!more) return;
+    stores_behind = full;
+  }
+}
+
+int compute_units() {
+  int device = 0, count = 0;
+  if (hipGetDevice(&device) != hipSuccess ||
+      hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || count <= 0)
+    return 256;
+  return count;
+}
+
+template <int TM, int TN>
+void set_tiles(LinearParams& prm) {
+  prm.tiles_m = (int)((prm.rows + TM - 1) / TM);
+  prm.tiles_n = prm.n / TN;
+  prm.num_tiles = prm.tiles_m * prm.tiles_n;
+  prm.group_m = 4;
+}
+
+template <typename T, int EPI, int TM, int TN>
+int launch_deep(LinearParams prm, hipStream_t stream) {
+  set_tiles<TM, TN>(prm);
+  const int cus = compute_units();
+  hipLaunchKernelGGL((linear_deep_kernel<T, EPI, TM, TN>), dim3(prm.num_tiles < cus ? prm.num_tiles : cus),
+                     dim3(256), 0, stream, prm);
+  return check_hip(hipGetLastError(), "linear kernel launch");
+}
+
+template <typename T, int EPI, int TM, int TN, int WM, int WN>
+int launch_ring(LinearParams prm, hipStream_t stream) {
+  set_tiles<TM, TN>(prm);
+  hipLaunchKernelGGL((linear_ring_kernel<T, EPI, TM, TN, WM, WN>), dim3(prm.num_tiles), dim3(WM * WN * 64), 0,
+                     stream, prm);
+  return check_hip(hipGetLastError(), "linear kernel launch");
+}
+
+}  // namespace
+
+template <typename T, int EPI>
+int launch_linear_tiles(LinearParams prm, hipStream_t stream) {
+  if (prm.seq_len > 1) {
+    // row / seq_len = (row * magic) >> (31 + l), 2^l >= seq_len, for rows below 2^31
+    int l = 1;
+    while ((1ull << l) < (unsigned long long)prm.seq_len) ++l;
+    prm.seq_magic = (uint32_t)((1ull << (31 + l)) / (uint32_t)prm.seq_len + 1);
+    prm.seq_shift = (uint32_t)(l - 1);
+  }
+  // The tile by the rounds that its grid takes on the CUs, each weighed by the
+  // time of a round against the 256 x 256 tile's.  Measured (bf16, us, plain
+  // Linear / with GELU), 256 x 256, 128 x 256 and the 128 x 128 ring:
+  //   777 x 1024 -> 4096     24.7 / 33.0    16.6 / 20.7    12.9 / 15.1
+  //   2000 x 1024 -> 4096    26.9 / 35.0    21.9 / 25.8    24.5 / 28.9
+  //   16384 x 2048 -> 512    43.3 / 51.1    35.8 / 40.2    42.3 / 45.8
+  //   16384 x 512 -> 2048    44.2 / 59.2    47.6 / 66.8    57.4 / 71.7
+  //   20002 x 1024 -> 3072    118 / 157      144 / 182      170 / 203
+  const int64_t cus = compute_units();
+  auto rounds = [&](int64_t tm, int64_t tn) { return ceil_div(ceil_div(prm.rows, tm) * (prm.n / tn), cus); };
+  const double deep256 = (double)rounds(256, 256);
+  const double deep128 = 0.6 * (double)rounds(128, 256);
+  const double ring128 = 0.38 * (double)rounds(128, 128);
+  if (ring128 <= deep128 && ring128 <= deep256) return launch_ring<T, EPI, 128, 128, 2, 2>(prm, stream);
+  if (deep128 <= deep256) return launch_deep<T, EPI, 128, 256>(prm, stream);
+  return launch_deep<T, EPI, 256, 256>(prm, stream);
+}
+
+template int launch_linear_tiles<bf16, kEpiRows>(LinearParams, hipStream_t);
+template int launch_linear_tiles<bf16, kEpiRowsGelu>(LinearParams, hipStream_t);
+template int launch_linear_tiles<bf16, kEpiHeads>(LinearParams, hipStream_t);
+template int launch_linear_tiles<bf16, kEpiHeadsSeqValue>(LinearParams, hipStream_t);
+template int launch_linear_tiles<f16, kEpiRows>(LinearParams, hipStream_t);
+template int launch_linear_tiles<f16, kEpiRowsGelu>(LinearParams, hipStream_t);
+template int launch_linear_tiles<f16, kEpiHeads>(LinearParams, hipStream_t);
+template int launch_linear_tiles<f16, kEpiHeadsSeqValue>(LinearParams, hipStream_t);
+
+}  // namespace sah

@@ -168,7 +168,7 @@ __global__ __launch_bounds__(kMlpThreads) void mlp_norm_kernel(MlpNormParams p) 
       }
       V4 out;
 #pragma unroll
-      for (int q = 0; q < 4; ++q) out[q] = from_f32<T>(gelu_exact(hacc[4 * g + q] + bv[q]));
+      for (int q = 0; q < 4; ++q) out[q] = from_f32<T>(fp32_result<T>(gelu_exact(hacc[4 * g + q] + bv[q])));
       *reinterpret_cast<V4*>(&h_lds[32 * rb + l32][hl]) = out;
     }
     __syncthreads();

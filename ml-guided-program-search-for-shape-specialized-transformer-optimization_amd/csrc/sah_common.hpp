@@ -112,8 +112,9 @@ __device__ __forceinline__ float gelu_exact(float v) {
   poly = fmaf(poly, t, 1.442729204e+00f);
   poly = fmaf(poly, t, -2.825748218e+00f);
   const float half_erfc = t * __builtin_amdgcn_exp2f(fmaf(-u, u, poly));
-  // v * Phi(v): v - v * erfc/2 for v >= 0, v * erfc/2 otherwise
-  return v >= 0.0f ? fmaf(-v, half_erfc, v) : v * half_erfc;
+  // v * Phi(v): v - v * erfc/2 for v >= 0, v * erfc/2 otherwise, as one fma
+  // on max(v, -0) (the -0 keeps the sign where the product underflows)
+  return fmaf(-fabsf(v), half_erfc, fmaxf(v, -0.0f));
 }
 
 // 16-byte global load/store of raw bits.

@@ -136,3 +136,62 @@ def test_ineligible_inputs_raise(gpu_device):
         prevalidated_hip_linear_exact_gelu(x, w, b)
     with pytest.raises(ValueError, match="launch"):
         prevalidated_hip_linear_exact_gelu(x, w, b, block_m=128)
+
+
+@pytest.mark.parametrize("k", [64, 128, 192, 320])
+@pytest.mark.parametrize(
+    "rows,n",
+    [(1, 256), (129, 512), (2047, 4096), (8191, 4096)],  # ring, ring, 128 x 256 and 256 x 256 tiles (256 CUs)
+)
+def test_every_tile_kernel_at_its_edges(gpu_device, rows, n, k):
+    """Each tile kernel with a partial last row tile and one to five K steps
+    (odd and even: both stages, all prefetch tails; several tiles per
+    workgroup for the largest), with and without GELU, bf16 and fp16, against
+    float64.  The K order is the same in every kernel, so rows computed alone
+    (the ring kernel) equal the same rows of the whole call bit for bit."""
+
+    from solution.kernels.ffn import prevalidated_hip_linear, prevalidated_hip_linear_exact_gelu
+
+    for dtype in (torch.bfloat16, torch.float16):
+        _, (xd, wd, bd) = _operands(rows, k, n, dtype, seed=rows + k, device=gpu_device)
+        exact = F.linear(xd.double(), wd.double(), bd.double())
+        for call, reference in ((prevalidated_hip_linear, exact), (prevalidated_hip_linear_exact_gelu, F.gelu(exact))):
+            with torch.inference_mode():
+                out, _ = call(xd, wd, bd)
+                head, _ = call(xd[:100].contiguous(), wd, bd)
+                tail, _ = call(xd[-77:].contiguous(), wd, bd)
+            torch.cuda.synchronize()
+            # one rounding of the result (unit roundoff 2^-8 at 8 significant
+            # bits, 2^-11 at 11; half the smallest fp16 step near zero), and
+            # fp32 accumulation of k products (k 2^-24 of sum |x| |w|, the
+            # activation's slope is below 2)
+            roundoff = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+            slack = k * 2.0**-24 * F.linear(xd.double().abs(), wd.double().abs(), bd.double().abs())
+            bound = roundoff * (reference.abs() + 2 * slack) + 2 * slack + 2.0**-25
+            err = (out.double() - reference).abs()
+            print(f"{call.__name__} {dtype} {rows}x{k}->{n}: max err {float(err.max()):.3g}", flush=True)
+            assert bool((err <= bound).all())
+            assert torch.equal(out[:100], head) and torch.equal(out[-77:], tail)
+
+
+def test_rows_beyond_the_tile_kernels_offsets(gpu_device):
+    """x rows more than 2^22 elements apart go to the register-staged kernel."""
+
+    from solution.kernels.ffn import prevalidated_hip_linear
+    from solution.kernels.hip import _library
+
+    rows, k, n, ldx = 3, 128, 256, (1 << 22) + 8
+    _, (xd, wd, bd) = _operands(rows, k, n, torch.bfloat16, seed=2, device=gpu_device)
+    far = torch.empty(rows, ldx, dtype=torch.bfloat16, device=gpu_device)
+    far[:, :k] = xd
+    y = torch.empty(rows, n, dtype=torch.bfloat16, device=gpu_device)
+    status = _library.load_library().sah_linear(
+        far.data_ptr(), wd.data_ptr(), bd.data_ptr(), y.data_ptr(), rows, k, n, ldx, n,
+        _library.dtype_code(torch.bfloat16), _library.SAH_ACTIVATION_NONE, 256, 256, 64, 8, 2,
+        _library.stream_handle(gpu_device),
+    )
+    _library.check_status(status, "sah_linear")
+    with torch.inference_mode():
+        expected, _ = prevalidated_hip_linear(xd, wd, bd)
+    torch.cuda.synchronize()
+    assert torch.equal(y, expected)
