@@ -350,8 +350,10 @@ int sah_qkv_launch_supported(int block_m, int block_n, int block_k, int num_warp
  *   update     = round_to(dtype, x weight^T + bias)   (fp32 accumulation, bias in fp32)
  *   residual   = round_to(dtype, value + update)
  *   normalized = round_to(dtype, norm(residual) * gamma + beta)
- * The update never reaches HBM.  The residual and norm arithmetic are those
- * of sah_residual_norm (statistics in fp32 over the rounded residual).
+ * Two launches on the stream (the projection leaves the rounded update in an
+ * output buffer, the norm reads it back in place); no workspace.  The residual
+ * and norm arithmetic are those of sah_residual_norm (statistics in fp32 over
+ * the rounded residual).
  *
  * Replaces the reference's
  *   _linear_residual_norm_kernel + triton_linear_residual_norm
@@ -364,8 +366,8 @@ int sah_qkv_launch_supported(int block_m, int block_n, int block_k, int num_warp
  * normalized not aliasing any input.  Shared dtype SAH_DTYPE_BF16 or
  * SAH_DTYPE_F16; norm_kind SAH_NORM_LAYER or SAH_NORM_RMS.  width 512 or
  * 1024, in_features a multiple of 64, x_row_stride a multiple of 8; tensors
- * 16-byte aligned, bias 8-byte.  Launch: block_rows = 65536 / width whole rows
- * per workgroup of num_warps = 8 wavefronts, see
+ * 16-byte aligned, bias 8-byte.  Launch: block_rows = 65536 / width, num_warps = 8
+ * (the one-kernel form's rows and wavefronts per workgroup), see
  * sah_linear_residual_norm_launch_supported().
  */
 int sah_linear_residual_norm(

@@ -1,9 +1,9 @@
 // Linear + residual add + LayerNorm / RMSNorm boundary for gfx950 (CDNA4).
 //
 // Same contract as the reference's fused linear boundary
-// (solution/kernels/boundary/triton_linear_residual_norm.py:34-109): the
+// (solution/kernels/boundary/triton_linear_residual_norm.py:34-109) on the
 // branch update of a block (the attention output projection, or the FFN
-// output projection) never reaches HBM.
+// output projection).
 //   update     = round_to(T, x W^T + b)          fp32 accumulation, bias in fp32
 //   residual   = round_to(T, value + update)
 //   normalized = round_to(T, norm(residual) * gamma + beta)
@@ -12,27 +12,37 @@
 // path does (the projection's output, then sah_residual_norm); the residual
 // and norm arithmetic are those of csrc/residual_norm.hip.
 //
-// MI355X formulation:
+// MI355X formulation: two launches on the caller's stream.  The projection
+// runs on the tile kernels (linear_tiles.hip) and leaves the rounded update in
+// one of the two output buffers; the fused norm kernel (residual_norm.hip)
+// then reads it back in place: a wavefront reads its whole row before it
+// writes it.  The update's round trip (4 bytes an element, mostly L2 and MALL
+// hits) costs far less than what keeping whole rows in one workgroup did:
+// a tile of 65536 / D rows by D columns streams all of W from L2 for every
+// 64 or 128 rows with uncoalesced 16-byte reads, and few rows leave most CUs
+// idle.  Measured on one box, one kernel -> two (bf16):
+//   16384 x 2048 -> 512     85 ->   50 us      64 x 2048 -> 512    69 -> 22 us
+//   20000 x 4096 -> 1024   558 ->  205 us     804 x 1024 -> 1024   71 -> 19 us
+//   200000 x 1024 -> 1024 1155 ->  672 us  200000 x 4096 -> 1024 3700 -> 1620 us
+//
+// The one-kernel form remains for outputs that both overlap an input, where
+// neither can hold the update.  In it:
 //  * One workgroup (8 wavefronts) owns BM = 65536 / D whole rows, so the row
 //    statistics never leave the workgroup.  Wave w computes output columns
 //    [w D/8, (w+1) D/8) of all BM rows: 8 accumulator blocks of 32 x 32
 //    (v_mfma_f32_32x32x16, computed transposed: update^T = W x^T).
-//  * W is read straight from global memory (L2: W is at most a few MB and is
-//    shared by every workgroup) into the MFMA A operand: each wave reads a
-//    disjoint slice, so staging it in LDS would buy no reuse.  Within each
-//    64-wide K step the K order is permuted (MFMA slice kk, lane half h takes
-//    k = 32 h + 8 kk .. +7) so every lane reads 64 contiguous bytes of its W
-//    row per step; x uses the same permutation when its fragments are read
-//    from LDS.  The W fragments of step s+1 are loaded into the registers of
-//    step s right after their MFMAs issue.
+//  * W is read straight from global memory (L2) into the MFMA A operand.
+//    Within each 64-wide K step the K order is permuted (MFMA slice kk, lane
+//    half h takes k = 32 h + 8 kk .. +7) so every lane reads 64 contiguous
+//    bytes of its W row per step; x uses the same permutation when its
+//    fragments are read from LDS.  The W fragments of step s+1 are loaded
+//    into the registers of step s right after their MFMAs issue.
 //  * x (shared by all 8 waves) goes through a double-buffered LDS stage
 //    (rows padded by 16 bytes: conflict-free 16-byte operand reads), one
 //    barrier per K step.
 //  * Epilogue: bias, one rounding, the bf16/fp16 update tile staged in the
 //    same LDS; then every wave normalizes whole rows exactly like the fused
-//    norm kernel (16-byte accesses, per-lane Welford state merged across the
-//    wavefront), reading the residual input and writing the residual and the
-//    normalized rows once.
+//    norm kernel.
 
 #include <cmath>
 
@@ -270,6 +280,12 @@ __global__ __launch_bounds__(kLnThreads) void linear_norm_kernel(LinearNormParam
   }
 }
 
+// Whether [a, a + a_bytes) and [b, b + b_bytes) share a byte (null: no).
+bool overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
+  const uintptr_t pa = reinterpret_cast<uintptr_t>(a), pb = reinterpret_cast<uintptr_t>(b);
+  return a != nullptr && b != nullptr && pa < pb + (uintptr_t)b_bytes && pb < pa + (uintptr_t)a_bytes;
+}
+
 template <typename T, int D>
 int launch_linear_norm(const LinearNormParams& prm, hipStream_t stream) {
   const int64_t blocks = (prm.rows + LnShape<D>::BM - 1) / LnShape<D>::BM;
@@ -332,6 +348,23 @@ extern "C" int sah_linear_residual_norm(const void* x, const void* weight, const
       (bias != nullptr && (reinterpret_cast<uintptr_t>(bias) & 7u) != 0))
     return fail(SAH_ERR_INVALID_ARGUMENT,
                 "sah_linear_residual_norm: tensors must be 16-byte aligned (bias 8-byte)");
+  // Two launches where an output can hold the update: one that overlaps no
+  // input (the reader of the next launch is the other output's too).
+  const int64_t row_bytes = width * 2, out_bytes = rows * row_bytes;
+  const int64_t x_bytes = ((rows - 1) * x_row_stride + in_features) * 2;
+  auto holds_update = [&](const void* out) {
+    return !overlap(out, out_bytes, x, x_bytes) && !overlap(out, out_bytes, value, out_bytes) &&
+           !overlap(out, out_bytes, weight, in_features * row_bytes) && !overlap(out, out_bytes, bias, row_bytes) &&
+           !overlap(out, out_bytes, gamma, row_bytes) && !overlap(out, out_bytes, beta, row_bytes);
+  };
+  void* update = holds_update(normalized) ? normalized : holds_update(residual) ? residual : nullptr;
+  if (update != nullptr) {
+    const int status = sah_linear(x, weight, bias, update, rows, in_features, width, x_row_stride, width, dtype,
+                                  SAH_ACTIVATION_NONE, 256, 256, 64, 8, 2, stream);
+    if (status != SAH_OK) return status;
+    return sah_residual_norm(value, update, gamma, beta, residual, normalized, rows, width, eps, dtype, dtype, dtype,
+                             dtype, norm_kind, 4, 4, stream);
+  }
   const int64_t blocks = (rows + block_rows - 1) / block_rows;
   if (blocks > INT32_MAX)
     return fail(SAH_ERR_UNSUPPORTED, "sah_linear_residual_norm: %lld rows is too many", (long long)rows);

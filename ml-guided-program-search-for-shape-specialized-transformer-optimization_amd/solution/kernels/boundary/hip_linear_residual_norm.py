@@ -10,15 +10,16 @@ ineligible", a failed launch RuntimeError "... execution failed").  The
 reference kernel (:34-109) multiplies a row block by the square projection
 weight, adds the bias, rounds the update to its fp16 branch dtype, adds it to
 the fp32 residual stream and normalizes, without writing the update.  This
-one (``sah_linear_residual_norm``, csrc/linear_norm.hip) does the same on a
-bf16 or fp16 stream: the update is rounded to the stream dtype, the residual
+one (``sah_linear_residual_norm``, csrc/linear_norm.hip) computes the same on a
+bf16 or fp16 stream in two launches (the update passes through an output
+buffer): the update is rounded to the stream dtype, the residual
 and the normalized rows are the stream dtype (there is no separate fp32
 final-boundary output: the stream is the model dtype), and the projection may
 be rectangular, so it serves both the attention output projection
 (in = width) and the FFN output projection (in = ffn_dim).
 
 Domain: width (d_model) 512 or 1024, in_features a multiple of 64; launch
-block_rows = 65536 / width whole rows per workgroup, num_warps = 8 (the
+block_rows = 65536 / width, num_warps = 8 (the
 reference's block_rows / num_warps launch fields, solution/config.py:327-355).
 """
 
@@ -139,8 +140,7 @@ def hip_linear_residual_norm(
     out: torch.Tensor | None = None,
 ) -> tuple[torch.Tensor, torch.Tensor, str]:
     """``residual = value + round(source @ weight.T + bias)``,
-    ``normalized = layer_norm(residual)``, without materializing the update
-    (reference: triton_linear_residual_norm, :197-245).  ``final_boundary``
+    ``normalized = layer_norm(residual)`` in one call (reference: triton_linear_residual_norm, :197-245).  ``final_boundary``
     is accepted for the reference's signature; on a same-dtype stream the
     final boundary's output has the stream dtype too.  ``out`` optionally
     receives the normalized tensor (e.g. a slice of a preallocated output)."""

@@ -1006,8 +1006,8 @@ class UserOptimizedTransformer(nn.Module):
     ) -> tuple[torch.Tensor, torch.Tensor]:
         """A branch's output projection fused with the residual add and the
         LayerNorm after it (reference: the triton_linear_residual_norm calls,
-        solution/transformer.py:699-725 and :1001-1033, here the gfx950
-        kernel); the update never reaches HBM."""
+        solution/transformer.py:699-725 and :1001-1033, here one call of
+        the gfx950 library)."""
 
         from .kernels.boundary.hip_linear_residual_norm import (
             HIP_LINEAR_RESIDUAL_NORM_BACKEND,

@@ -192,3 +192,38 @@ def test_ineligible_inputs_raise(gpu_device):
         with pytest.raises(RuntimeError, match="output buffer"):
             hip_linear_residual_norm(x, w, None, v, ln, block_rows=64, num_warps=8, out=torch.empty_like(v).float())
     assert not can_use_hip_linear_residual_norm(x, w, None, v, ln, block_rows=64, num_warps=8)  # grad enabled
+
+
+@pytest.mark.parametrize("residual_on,normalized_on", [
+    (None, "value"),      # the update waits in the residual buffer
+    ("value", None),      # ... in the normalized buffer
+    ("value", "x"),       # neither can hold it: the one-kernel form
+])
+def test_outputs_over_inputs_through_the_c_abi(gpu_device, residual_on, normalized_on):
+    """Outputs written over inputs give the separate buffers' results bit for
+    bit (exact integer products, so the accumulation order does not show)."""
+
+    from solution.kernels.boundary import block_rows_for, hip_linear_residual_norm
+    from solution.kernels.hip import _library
+
+    width, rows, dtype = 512, 300, torch.bfloat16
+    g = torch.Generator().manual_seed(11)
+    x = torch.randint(-2, 3, (1, rows, width), generator=g).to(dtype).to(gpu_device)
+    w = (torch.randint(-2, 3, (width, width), generator=g).float() / 16).to(dtype).to(gpu_device)
+    b = torch.randn(width, generator=g).to(dtype).to(gpu_device)
+    value = torch.randn(1, rows, width, generator=g).to(dtype).to(gpu_device)
+    ln = _layer_norm(width, dtype, gpu_device, seed=3)
+    with torch.inference_mode():
+        r_ref, y_ref, _ = hip_linear_residual_norm(
+            x, w, b, value, ln, block_rows=block_rows_for(width), num_warps=8)
+    buffers = {"value": value, "x": x, None: None}
+    residual = buffers[residual_on] if residual_on else torch.empty_like(value)
+    normalized = buffers[normalized_on] if normalized_on else torch.empty_like(value)
+    status = _library.load_library().sah_linear_residual_norm(
+        x.data_ptr(), w.data_ptr(), b.data_ptr(), value.data_ptr(), ln.weight.data_ptr(), ln.bias.data_ptr(),
+        residual.data_ptr(), normalized.data_ptr(), rows, width, width, width, ln.eps, _library.dtype_code(dtype),
+        _library.SAH_NORM_LAYER, block_rows_for(width), 8, _library.stream_handle(gpu_device),
+    )
+    _library.check_status(status, "sah_linear_residual_norm")
+    torch.cuda.synchronize()
+    assert torch.equal(residual, r_ref) and torch.equal(normalized, y_ref)
