@@ -29,6 +29,7 @@ SOURCES = (
     "residual_norm.hip",
     "attention_fwd.hip",
     "attention_scaled.hip",
+    "attention_f32.hip",
     "linear_gelu.hip",
     "linear_tiles.hip",
     "gelu.hip",

@@ -639,3 +639,31 @@ def test_fp32_attention_scale_sign_and_packed_views(gpu_device, scale):
     torch.cuda.synchronize(gpu_device)
     reference = _to_bsd(_oracle(q, k, v, scale))
     _assert_parity(reference, output, torch.float32, f"fp32 packed scale {scale}")
+
+
+@pytest.mark.parametrize(
+    "batch,heads,seq",
+    [(1, 3, 31), (1, 3, 32), (2, 1, 33), (1, 8, 127), (1, 8, 128), (1, 5, 129), (1, 2, 2049)],
+)
+def test_fp32_attention_block_edges_against_float64(gpu_device, batch, heads, seq):
+    """Sequences about the fp32 kernel's 32-key blocks and its four-way key
+    split (waves with no block, one block, a partial one), against float64.
+
+    Bound: a score's fp32 error is at most 64 2^-24 sum |q k| scale = d; it
+    moves a weight by a factor e^(+-2 d), so an output by 2 d max |v|; summing
+    at most seq weights and products in fp32 adds (seq + 8) 2^-24 max |v|."""
+
+    print(f"fp32 edges {(batch, heads, seq)}", flush=True)
+    q, k, v = (t.to(gpu_device) for t in _inputs(batch, heads, seq, dtype=torch.float32, seed=seq + heads))
+    module = _attention_module()
+    with torch.inference_mode():
+        output, _ = module.hip_streaming_dh64_causal_attention_bsd(q, k, v)
+    torch.cuda.synchronize(gpu_device)
+    scores = q.double() @ k.double().transpose(-1, -2).contiguous() / 8
+    future = torch.ones(seq, seq, dtype=torch.bool, device=gpu_device).triu(1)
+    expected = _to_bsd(torch.softmax(scores.masked_fill(future, float("-inf")), dim=-1) @ v.double())
+    d = 64 * 2.0**-24 * float((q.double().abs() @ k.double().abs().transpose(-1, -2).contiguous()).max()) / 8
+    bound = float(v.abs().max()) * (2.1 * d + (seq + 8) * 2.0**-24)
+    error = float((output.double() - expected).abs().max())
+    print(f"  max error {error:.3g}, bound {bound:.3g}", flush=True)
+    assert error <= bound
