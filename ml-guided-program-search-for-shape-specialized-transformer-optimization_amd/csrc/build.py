@@ -32,6 +32,7 @@ SOURCES = (
     "attention_f32.hip",
     "linear_gelu.hip",
     "linear_tiles.hip",
+    "linear_f32.hip",
     "gelu.hip",
     "linear_norm.hip",
     "mlp_norm.hip",

@@ -1,0 +1,109 @@
+"""The small fp32 Linear layers of a model on the gfx950 kernel.
+
+Counterpart of the reference's ``nn.Linear`` projections
+(solution/transformer.py:291-353) for fp32 models of few rows: the same
+operands and result (``sah_linear_f32``, csrc/linear_f32.hip).  ``project``
+takes a call that it is measured faster on and returns None for every other
+one, which then runs ``F.linear``.
+"""
+
+from __future__ import annotations
+
+import torch
+from torch import nn
+
+from ..hip._library import (
+    check_status,
+    is_gfx950,
+    load_library,
+    stream_handle,
+)
+
+# The 32 x 32 tiles that one round of the 256 CUs takes, and the K whose row
+# segments the loads read well (GPU time in us, library / this kernel):
+#   256 x 256 -> 256     63 / 4.8     512 x 256 -> 768     5.8 /  7.8
+#   256 x 256 -> 1024   5.7 / 5.1    1024 x 256 -> 1024    8.0 / 13.8
+#   100 x 128 -> 128   11.4 / 3.9     256 x 1024 -> 256    5.8 / 10.0
+# A call also costs the host about half of F.linear's.  (The 16-bit tile
+# kernels were tried here too: at 16384 x 512 -> 1536 and 512 -> 512 they are
+# 4-9% faster than the library alone, but the forward of that stack measured
+# the same, 835 us.)
+_MAX_TILES = 256
+_MAX_IN = 384
+
+
+def _serves(rows: int, in_features: int, out_features: int, dtype: torch.dtype) -> bool:
+    """The rule on sizes and types."""
+
+    return (
+        dtype == torch.float32
+        and in_features <= _MAX_IN
+        and in_features % 128 == 0
+        and out_features % 32 == 0
+        and (rows + 31) // 32 * (out_features // 32) <= _MAX_TILES
+    )
+
+
+def _is_plain(module: nn.Linear, value: torch.Tensor) -> bool:
+    """Whether calling ``module`` is no more than one F.linear on plain
+    tensors: nothing observes, differentiates, casts or traces the call."""
+
+    if torch.compiler.is_compiling() or torch.jit.is_tracing():
+        return False
+    if torch.is_grad_enabled() or torch.is_autocast_enabled("cuda"):
+        return False
+    if type(value) is not torch.Tensor or type(module.weight) not in (nn.Parameter, torch.Tensor):
+        return False
+    if module.bias is not None and type(module.bias) not in (nn.Parameter, torch.Tensor):
+        return False
+    if module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__:
+        return False
+    registry = nn.modules.module
+    if registry._global_forward_hooks or registry._global_forward_pre_hooks:
+        return False
+    return not (
+        torch._C._len_torch_dispatch_stack()
+        or torch._C._len_torch_function_stack()
+        or torch._C._functorch.peek_interpreter_stack() is not None
+    )
+
+
+def project(module: nn.Linear, value: torch.Tensor) -> torch.Tensor | None:
+    """``module(value)`` on the gfx950 kernel, or None where they do not
+    serve the call (size, type, layout, or a call that something observes)."""
+
+    weight, bias = module.weight, module.bias
+    dtype = value.dtype
+    out_features, in_features = weight.shape
+    if not value.is_cuda or value.ndim < 2 or value.shape[-1] != in_features:
+        return None
+    rows = value.numel() // in_features
+    if rows == 0 or not _serves(rows, in_features, out_features, dtype) or not _is_plain(module, value):
+        return None
+    if weight.dtype != dtype or weight.device != value.device or not (value.is_contiguous() and weight.is_contiguous()):
+        return None
+    pointers = (value.data_ptr(), weight.data_ptr(), 0 if bias is None else bias.data_ptr())
+    if (pointers[0] | pointers[1] | pointers[2]) % 16:
+        return None
+    if bias is not None and (bias.dtype != dtype or bias.device != value.device or not bias.is_contiguous()):
+        return None
+    if not is_gfx950(value.device):
+        return None
+    output = torch.empty((*value.shape[:-1], out_features), device=value.device, dtype=dtype)
+    status = load_library().sah_linear_f32(
+        pointers[0],
+        pointers[1],
+        pointers[2] or None,
+        output.data_ptr(),
+        rows,
+        in_features,
+        out_features,
+        in_features,
+        out_features,
+        stream_handle(value.device),
+    )
+    check_status(status, "sah_linear_f32")
+    return output
+
+
+__all__ = ["project"]

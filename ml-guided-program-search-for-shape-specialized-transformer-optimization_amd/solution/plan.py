@@ -194,6 +194,10 @@ class ExecutionPlan:
         return self.config.config_id
 
     @property
+    def uses_hip_attention(self) -> bool:
+        return self.attention_backend is AttentionBackend.HIP_STREAMING_DH64
+
+    @property
     def use_cuda_graph(self) -> bool:
         return self.runtime_backend is RuntimeBackend.CUDA_GRAPH
 

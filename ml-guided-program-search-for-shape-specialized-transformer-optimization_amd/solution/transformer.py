@@ -265,10 +265,22 @@ class _FP16ShadowLinear(nn.Linear):
         self._fp16_shadow_weight = None
         self._fp16_shadow_bias = None
 
-    def forward_backend(self, value: torch.Tensor, backend: ProjectionBackend) -> torch.Tensor:
+    def forward_backend(
+        self, value: torch.Tensor, backend: ProjectionBackend, *, hip: bool = False
+    ) -> torch.Tensor:
+        """The projection by ``backend``.  ``hip`` (the programs on the HIP
+        attention): a small fp32 projection may run on the gfx950 kernel, at
+        the sizes where it beats the library GEMM."""
+
         if backend is ProjectionBackend.INPUT_DTYPE:
             if value.dtype != self.weight.dtype:
                 value = value.to(self.weight.dtype)
+            if hip:
+                from .kernels.projection.hip_linear import project
+
+                output = project(self, value)
+                if output is not None:
+                    return output
             return self(value)
         if backend is ProjectionBackend.AUTOCAST_FP16:
             with torch.autocast(device_type=value.device.type, dtype=torch.float16, enabled=True):
@@ -359,7 +371,7 @@ class _SelfAttention(nn.Module):
                 observation.qkv_materializations.append(plan.qkv_materialization.value)
                 observation.qkv_launches.append(_launch_dict(plan.qkv_launch))
         else:
-            packed = self.qkv_proj.forward_backend(value, plan.qkv_projection_backend)
+            packed = self.qkv_proj.forward_backend(value, plan.qkv_projection_backend, hip=plan.uses_hip_attention)
             qkv_dtype = packed.dtype
             query, key, projected = split_qkv(
                 packed,
@@ -422,7 +434,9 @@ class _SelfAttention(nn.Module):
                 f"attention bridge {plan.attention_output_bridge.value} is not executable here"
             )
         output = (
-            self.out_proj.forward_backend(context, plan.attention_output_projection_backend)
+            self.out_proj.forward_backend(
+                context, plan.attention_output_projection_backend, hip=plan.uses_hip_attention
+            )
             if project
             else context
         )
@@ -527,7 +541,9 @@ class _TransformerBlock(nn.Module):
             launch = plan.ffn_launch
             if launch is None:
                 raise RuntimeError("HIP Exact-GELU plan is missing launch parameters")
-            projected = self.ffn_in.forward_backend(normalized, plan.ffn_input_projection_backend)
+            projected = self.ffn_in.forward_backend(
+                normalized, plan.ffn_input_projection_backend, hip=plan.uses_hip_attention
+            )
             input_compute_dtype = _dtype_name(projected.dtype)
             # in place: the projection is a temporary of this block
             hidden, marker = prevalidated_hip_exact_gelu(
@@ -537,13 +553,19 @@ class _TransformerBlock(nn.Module):
                 marker, expected_marker=HIP_EXACT_GELU_BACKEND, planned_backend=plan.ffn_backend.value
             )
         else:
-            projected = self.ffn_in.forward_backend(normalized, plan.ffn_input_projection_backend)
+            projected = self.ffn_in.forward_backend(
+                normalized, plan.ffn_input_projection_backend, hip=plan.uses_hip_attention
+            )
             input_compute_dtype = _dtype_name(projected.dtype)
             if plan.ffn_activation_output_dtype == "float32":
                 projected = projected.float()
             hidden = F.gelu(projected, approximate="none")
         update = (
-            self.ffn_out.forward_backend(hidden, plan.ffn_output_projection_backend) if project else hidden
+            self.ffn_out.forward_backend(
+                hidden, plan.ffn_output_projection_backend, hip=plan.uses_hip_attention
+            )
+            if project
+            else hidden
         )
         if observation is not None:
             observation.ffn_input_projection_backends.append(plan.ffn_input_projection_backend.value)

@@ -195,3 +195,62 @@ def test_rows_beyond_the_tile_kernels_offsets(gpu_device):
         expected, _ = prevalidated_hip_linear(xd, wd, bd)
     torch.cuda.synchronize()
     assert torch.equal(y, expected)
+
+
+@pytest.mark.parametrize("rows", [1, 31, 33, 256])
+@pytest.mark.parametrize("k,n", [(128, 32), (256, 256), (384, 96), (1024, 64)])
+def test_fp32_linear_at_its_edges(gpu_device, rows, k, n):
+    """sah_linear_f32 about its 32 x 32 tiles and 32-wide load steps, with
+    padded rows on both sides, against float64: k products and sums in fp32,
+    (k + 4) 2^-24 of sum |x| |w| + |b|."""
+
+    from solution.kernels.hip import _library
+
+    g = torch.Generator().manual_seed(rows + k + n)
+    ldx, ldy = k + 4, n + 8
+    xs = torch.full((rows, ldx), float("nan"))
+    xs[:, :k] = torch.randn(rows, k, generator=g)
+    w, b = torch.randn(n, k, generator=g).to(gpu_device), torch.randn(n, generator=g).to(gpu_device)
+    xs = xs.to(gpu_device)
+    for bias in (b, None):
+        y = torch.full((rows + 2, ldy), -7.0, device=gpu_device)
+        status = _library.load_library().sah_linear_f32(
+            xs.data_ptr(), w.data_ptr(), None if bias is None else bias.data_ptr(), y.data_ptr(), rows, k, n, ldx,
+            ldy, _library.stream_handle(gpu_device),
+        )
+        _library.check_status(status, "sah_linear_f32")
+        torch.cuda.synchronize()
+        x = xs[:, :k].double()
+        expected = F.linear(x, w.double(), None if bias is None else bias.double())
+        size = F.linear(x.abs(), w.double().abs(), None if bias is None else bias.double().abs())
+        error = (y[:rows, :n].double() - expected).abs()
+        print(f"fp32 linear {rows}x{k}->{n}: max err {float(error.max()):.3g}", flush=True)
+        assert bool((error <= (k + 4) * 2.0**-24 * size).all())
+        assert bool((y[:rows, n:] == -7.0).all()) and bool((y[rows:] == -7.0).all())
+
+
+def test_model_projection_takes_what_it_serves(gpu_device):
+    """project() against F.linear: the calls it serves agree to fp32 rounding, and
+    every call that something observes or casts, or that the rule or the
+    layout leaves out, is refused."""
+
+    from solution.kernels.projection.hip_linear import project
+
+    rows, k, n, dtype = 100, 256, 192, torch.float32
+    linear = torch.nn.Linear(k, n, device=gpu_device, dtype=dtype)
+    value = torch.randn(1, rows, k, device=gpu_device, dtype=dtype)
+    with torch.no_grad():
+        out = project(linear, value)
+        exact = F.linear(value.double(), linear.weight.double(), linear.bias.double())
+        size = F.linear(value.double().abs(), linear.weight.double().abs(), linear.bias.double().abs())
+        bound = (k + 4) * 2.0**-24 * size
+        assert out.shape == (1, rows, n) and bool(((out.double() - exact).abs() <= bound).all())
+        assert project(linear, torch.randn(1, rows, k + 8, device=gpu_device, dtype=dtype)[..., :k]) is None
+        assert project(linear, value.cpu()) is None
+        with torch.autocast("cuda", dtype=torch.float16):
+            assert project(linear, value) is None
+        handle = linear.register_forward_hook(lambda *_: None)
+        assert project(linear, value) is None
+        handle.remove()
+        assert project(linear, value) is not None
+    assert project(linear, value) is None  # grad enabled

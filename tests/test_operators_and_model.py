@@ -144,3 +144,20 @@ def test_hip_config_is_rejected_on_cpu_without_fallback():
     model = _model(config, default_init_weights(config, seed=2))
     with pytest.raises(ConfigRejectedError, match="program.attention"):
         model.configure_execution(config=hip_config())
+
+
+def test_model_projection_rule():
+    """Which Linear calls the fp32 kernel serves, by size and type; none off
+    the GPU."""
+
+    from solution.kernels.projection.hip_linear import _serves, project
+
+    f32 = torch.float32
+    assert _serves(256, 256, 1024, f32) and _serves(1, 384, 32, f32) and _serves(8192, 128, 32, f32)
+    for sizes in [(257, 256, 1024), (256, 512, 256), (256, 192, 256), (256, 256, 200)]:
+        assert not _serves(*sizes, f32), sizes
+    for dtype in (torch.float64, torch.bfloat16, torch.float16):
+        assert not _serves(64, 256, 256, dtype)
+    linear = torch.nn.Linear(256, 256)
+    with torch.no_grad():
+        assert project(linear, torch.zeros(2, 8, 256)) is None
