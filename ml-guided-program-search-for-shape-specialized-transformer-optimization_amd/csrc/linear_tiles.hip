@@ -14,6 +14,9 @@
 //   65536 x 2048 -> 8192    2567 -> 1710 us (1286 TFLOP/s), GELU 2786 -> 1960 us
 //   20002 x 1024 -> 3072     154 ->  118 us, GELU 179 -> 157 us
 //   777 x 1024 -> 4096        36 ->   13 us, GELU  44 ->  15 us
+//   64 x 4096 -> 1024        102 ->   20 us
+// Few rows take smaller tiles on more CUs: one CU loads about 60 GB/s, and a
+// tile's K steps wait for that.
 // Tried and slower at 65536 x 2048 -> 8192: two groups of four waves half a
 // step apart on 128 x 64 wave tiles (1983 us); stores of a tile spread over
 // the next tile's main loop from registers (1790 us: 32-byte segments and
@@ -80,7 +83,7 @@ __device__ __forceinline__ void store_wave(const LinearParams& p, unsigned char*
   asm volatile("" : "+v"(lane));  // addresses formed here, not kept over the main loop
   const int l32 = lane & 31;
   const int half = lane >> 5;
-  auto slot = [](int row, int chunk) { return chunk ^ (CPR == 16 ? row & 15 : (row >> 1) & (CPR - 1)); };
+  auto slot = [](int row, int chunk) { return chunk ^ ((row >> (CPR == 16 ? 0 : CPR == 8 ? 1 : 2)) & (CPR - 1)); };
 
   const int chunk = lane % CPR;
   const int col = n_wave + chunk * 8;
@@ -210,11 +213,11 @@ __device__ __forceinline__ void clear(f32x16 (&acc)[NI][NJ]) {
       for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.0f;
 }
 
-// One tile per workgroup, the four-stage ring.
-template <typename T, int EPI, int TM, int TN, int WM, int WN>
-__global__ __launch_bounds__(WM * WN * 64) void linear_ring_kernel(LinearParams p) {
-  typedef GemmTile<T, TM, TN, WM, WN> Tile;
-  constexpr uint32_t kStageBytes = Tile::RING * (Tile::XSTAGE + Tile::WSTAGE);
+// One tile per workgroup of 2 x 2 waves, a ring of R stages.
+template <typename T, int EPI, int TM, int TN, int R>
+__global__ __launch_bounds__(256, 1) void linear_ring_kernel(LinearParams p) {
+  typedef GemmTile<T, TM, TN, 2, 2> Tile;
+  constexpr uint32_t kStageBytes = R * (Tile::XSTAGE + Tile::WSTAGE);
   constexpr uint32_t kAreaBytes = 32 * Tile::COLS * sizeof(T);
   __shared__ __attribute__((aligned(16))) unsigned char smem[kStageBytes + Tile::WAVES * kAreaBytes];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -227,17 +230,17 @@ __global__ __launch_bounds__(WM * WN * 64) void linear_ring_kernel(LinearParams 
   const int64_t m0 = (int64_t)tile_m * TM;
   const int n0 = tile_n * TN;
   Tile tile;
-  tile.init(smem, Tile::RING * Tile::XSTAGE);
+  tile.init(smem, R * Tile::XSTAGE);
   const int64_t left = p.rows - m0;
   tile.operands(static_cast<const T*>(p.x) + m0 * p.x_ld, p.x_ld, left < TM ? (int)left : TM,
                 static_cast<const T*>(p.w) + (int64_t)n0 * p.k, p.k);
-  const int n_wave = n0 + wave % WN * Tile::COLS;
+  const int n_wave = n0 + wave % 2 * Tile::COLS;
   WaveBias<T, Tile::NI> bias;
   bias.load(static_cast<const T*>(p.bias), n_wave);
   f32x16 acc[Tile::NI][Tile::NJ];
   clear(acc);
-  tile.ring(smem, p.k / kTileK, acc);
-  store_wave<T, EPI>(p, smem + kStageBytes + wave * kAreaBytes, m0 + wave / WN * Tile::ROWS, n_wave, bias,
+  tile.template ring<R>(smem, p.k / kTileK, acc);
+  store_wave<T, EPI>(p, smem + kStageBytes + wave * kAreaBytes, m0 + wave / 2 * Tile::ROWS, n_wave, bias,
                      acc, [](int) {});
 }
 
@@ -338,11 +341,10 @@ int launch_deep(LinearParams prm, hipStream_t stream) {
   return check_hip(hipGetLastError(), "linear kernel launch");
 }
 
-template <typename T, int EPI, int TM, int TN, int WM, int WN>
+template <typename T, int EPI, int TM, int TN, int R>
 int launch_ring(LinearParams prm, hipStream_t stream) {
   set_tiles<TM, TN>(prm);
-  hipLaunchKernelGGL((linear_ring_kernel<T, EPI, TM, TN, WM, WN>), dim3(prm.num_tiles), dim3(WM * WN * 64), 0,
-                     stream, prm);
+  hipLaunchKernelGGL((linear_ring_kernel<T, EPI, TM, TN, R>), dim3(prm.num_tiles), dim3(256), 0, stream, prm);
   return check_hip(hipGetLastError(), "linear kernel launch");
 }
 
@@ -365,12 +367,29 @@ int launch_linear_tiles(LinearParams prm, hipStream_t stream) {
   //   16384 x 2048 -> 512    43.3 / 51.1    35.8 / 40.2    42.3 / 45.8
   //   16384 x 512 -> 2048    44.2 / 59.2    47.6 / 66.8    57.4 / 71.7
   //   20002 x 1024 -> 3072    118 / 157      144 / 182      170 / 203
+  // The tile by an estimate of its time in us: rounds of its grid on the CUs,
+  // each of K / 64 steps and an epilogue.  A step costs what one CU loads
+  // ((TM + TN) rows of 128 bytes at about 60 GB/s) or multiplies; two 64 x 64
+  // workgroups share a CU.  Measured (bf16 Linear, us), 64 x 64, 128 x 128,
+  // 128 x 256 and 256 x 256:
+  //   64 x 4096 -> 1024     19.9   35.8   43.8   68.0
+  //   800 x 2048 -> 512     11.8   19.9   25.1   38.4
+  //   777 x 1024 -> 4096    16.3   13.4   16.5   24.3
+  //   2000 x 1024 -> 3072   25.5   24.0   18.8   25.9
+  //   6000 x 1024 -> 4096   93.7   73.5   57.5   55.6
+  //   16384 x 2048 -> 512            42     36     43
+  //   20002 x 1024 -> 3072          170    144    118
   const int64_t cus = compute_units();
-  auto rounds = [&](int64_t tm, int64_t tn) { return ceil_div(ceil_div(prm.rows, tm) * (prm.n / tn), cus); };
-  const double deep256 = (double)rounds(256, 256);
-  const double deep128 = 0.6 * (double)rounds(128, 256);
-  const double ring128 = 0.38 * (double)rounds(128, 128);
-  if (ring128 <= deep128 && ring128 <= deep256) return launch_ring<T, EPI, 128, 128, 2, 2>(prm, stream);
+  const double steps = (double)(prm.k / kTileK);
+  auto tiles = [&](int64_t tm, int64_t tn) { return ceil_div(prm.rows, tm) * (prm.n / tn); };
+  auto rounds = [&](int64_t tm, int64_t tn) { return (double)ceil_div(tiles(tm, tn), cus); };
+  const double t64 = (double)tiles(64, 64) / (double)(2 * cus);
+  const double ring64 = t64 <= 0.5 ? steps * 0.28 + 1.0 : (t64 < 1.0 ? 1.0 : t64) * (steps * 0.39 + 1.5);
+  const double ring128 = rounds(128, 128) * (steps * 0.54 + 2.5);
+  const double deep128 = rounds(128, 256) * (steps * 0.66 + 4.0);
+  const double deep256 = rounds(256, 256) * (steps * 1.03 + 7.0);
+  if (ring64 <= ring128 && ring64 <= deep128 && ring64 <= deep256) return launch_ring<T, EPI, 64, 64, 4>(prm, stream);
+  if (ring128 <= deep128 && ring128 <= deep256) return launch_ring<T, EPI, 128, 128, 4>(prm, stream);
   if (deep128 <= deep256) return launch_deep<T, EPI, 128, 256>(prm, stream);
   return launch_deep<T, EPI, 256, 256>(prm, stream);
 }

@@ -141,14 +141,15 @@ def test_ineligible_inputs_raise(gpu_device):
 @pytest.mark.parametrize("k", [64, 128, 192, 320])
 @pytest.mark.parametrize(
     "rows,n",
-    [(1, 256), (129, 512), (2047, 4096), (8191, 4096)],  # ring, ring, 128 x 256 and 256 x 256 tiles (256 CUs)
+    # 64 x 64 (twice), 128 x 128, 128 x 256 and 256 x 256 tiles (256 CUs)
+    [(1, 256), (129, 512), (777, 4096), (2047, 4096), (8191, 4096)],
 )
 def test_every_tile_kernel_at_its_edges(gpu_device, rows, n, k):
     """Each tile kernel with a partial last row tile and one to five K steps
     (odd and even: both stages, all prefetch tails; several tiles per
     workgroup for the largest), with and without GELU, bf16 and fp16, against
     float64.  The K order is the same in every kernel, so rows computed alone
-    (the ring kernel) equal the same rows of the whole call bit for bit."""
+    (the 64 x 64 tiles) equal the same rows of the whole call bit for bit."""
 
     from solution.kernels.ffn import prevalidated_hip_linear, prevalidated_hip_linear_exact_gelu
 
