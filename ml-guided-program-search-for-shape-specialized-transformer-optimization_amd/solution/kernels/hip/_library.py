@@ -203,6 +203,9 @@ _GFX950_BY_INDEX: dict[int, bool] = {}
 def is_gfx950(device: torch.device) -> bool:
     """Whether ``device`` is a CDNA4 (gfx950) GPU visible to torch."""
 
+    known = _GFX950_BY_INDEX.get(device.index)  # cuda indices only are recorded
+    if known is not None and device.type == "cuda":
+        return known
     if device.type != "cuda" or torch.version.hip is None:
         return False
     if not _GFX950_BY_INDEX and not torch.cuda.is_available():

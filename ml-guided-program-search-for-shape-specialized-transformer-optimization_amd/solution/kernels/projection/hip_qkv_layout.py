@@ -66,10 +66,10 @@ def launch_config_is_valid(block_m: int, block_n: int, block_k: int, num_warps: 
     """The launch the gfx950 kernel implements (the C library's own table)."""
 
     values = (block_m, block_n, block_k, num_warps)
-    if any(isinstance(value, bool) or not isinstance(value, int) for value in values):
-        return False
-    if library_available():
-        return bool(load_library().sah_qkv_launch_supported(*values))
+    for value in values:
+        if isinstance(value, bool) or not isinstance(value, int):
+            return False
+    # the library's table has this one row (checked against it in the tests)
     return values == (DEFAULT_BLOCK_M, DEFAULT_BLOCK_N, DEFAULT_BLOCK_K, DEFAULT_NUM_WARPS)
 
 
@@ -371,17 +371,11 @@ def hip_qkv_native_bhsd(
         num_warps=num_warps,
     ):
         raise RuntimeError("HIP QKV native-layout projection is ineligible")
-    return prevalidated_hip_qkv_native_bhsd(
-        hidden_states,
-        weight,
-        bias,
-        num_heads=num_heads,
-        block_m=block_m,
-        block_n=block_n,
-        block_k=block_k,
-        num_warps=num_warps,
-        value_layout=value_layout,
-    )
+    if value_layout not in VALUE_LAYOUTS:
+        raise ValueError(f"unknown value layout {value_layout!r}; expected one of {sorted(VALUE_LAYOUTS)}")
+    return _launch(
+        hidden_states, None, weight, bias, num_heads, (block_m, block_n, block_k, num_warps), value_layout
+    ) + (HIP_QKV_NATIVE_BHSD_BACKEND,)
 
 
 __all__ = [

@@ -18,6 +18,7 @@ its workspace.
 
 from __future__ import annotations
 
+import functools
 import math
 
 import torch
@@ -35,6 +36,7 @@ from ..kernels.hip._library import (
 HIP_STREAMING_DH64_CAUSAL_ATTENTION_BSD_BACKEND = "hip_streaming_dh64_causal_attention_bsd"
 _HEAD_DIM = 64
 _SUPPORTED_DTYPES = frozenset({torch.bfloat16, torch.float16, torch.float32})
+_DEFAULT_SCALE = 1.0 / math.sqrt(_HEAD_DIM)
 _DEFAULT_BLOCK_M = 128
 _DEFAULT_BLOCK_N = 64
 _DEFAULT_NUM_WARPS = 4
@@ -62,20 +64,25 @@ def launch_config_is_valid(
     """
 
     values = (block_m, block_n, num_warps, num_stages)
-    return bool(
-        not any(isinstance(value, bool) for value in values)
-        and all(isinstance(value, int) for value in values)
-        and block_m in SUPPORTED_BLOCK_M
-        and block_n in SUPPORTED_BLOCK_N
-        and num_warps in SUPPORTED_NUM_WARPS
-        and num_stages in SUPPORTED_NUM_STAGES
-        and (
-            # three stages select the software-pipelined kernel (4 waves, 128 rows)
-            (block_m == 128 and num_warps == 4)
-            if num_stages == 3
-            else block_m in (32 * num_warps, 64 * num_warps)
-        )
+    for value in values:
+        if isinstance(value, bool) or not isinstance(value, int):
+            return False
+    return values in _LAUNCHES
+
+
+# three stages select the software-pipelined kernel (4 waves, 128 rows)
+_LAUNCHES = frozenset(
+    (block_m, block_n, num_warps, num_stages)
+    for block_m in SUPPORTED_BLOCK_M
+    for block_n in SUPPORTED_BLOCK_N
+    for num_warps in SUPPORTED_NUM_WARPS
+    for num_stages in SUPPORTED_NUM_STAGES
+    if (
+        (block_m == 128 and num_warps == 4)
+        if num_stages == 3
+        else block_m in (32 * num_warps, 64 * num_warps)
     )
+)
 
 
 def _validate_launch_config(
@@ -97,6 +104,13 @@ def _strides(tensor: torch.Tensor) -> tuple[int, ...]:
     )
 
 
+@functools.lru_cache(maxsize=256)
+def _workspace_bytes(batch: int, heads: int, seq_len: int, head_dim: int, v_ss: int, v_sd: int, code: int) -> int:
+    """The library's workspace size, a function of these sizes alone."""
+
+    return int(load_library().sah_causal_attention_workspace_bytes(batch, heads, seq_len, head_dim, v_ss, v_sd, code))
+
+
 def _launch(
     query: torch.Tensor,
     key: torch.Tensor,
@@ -113,9 +127,8 @@ def _launch(
         (batch, seq_len, heads * head_dim), dtype=query.dtype, device=query.device
     )
     code = dtype_code(query.dtype)
-    workspace_bytes = library.sah_causal_attention_workspace_bytes(
-        batch, heads, seq_len, head_dim, *_strides(value)[2:], code
-    )
+    v_strides = _strides(value)
+    workspace_bytes = _workspace_bytes(batch, heads, seq_len, head_dim, v_strides[2], v_strides[3], code)
     workspace = (
         torch.empty(workspace_bytes, dtype=torch.uint8, device=query.device)
         if workspace_bytes
@@ -123,7 +136,6 @@ def _launch(
     )
     q_strides = _strides(query)
     k_strides = _strides(key)
-    v_strides = _strides(value)
     status = library.sah_causal_attention_bsd(
         query.data_ptr(),
         key.data_ptr(),
@@ -136,8 +148,8 @@ def _launch(
         *q_strides[:3],
         *k_strides[:3],
         *v_strides,
-        output.stride(0),
-        output.stride(1),
+        seq_len * heads * head_dim,
+        heads * head_dim,
         float(scale),
         code,
         block_m,
@@ -237,11 +249,13 @@ def can_use_hip_streaming_dh64_causal_attention(
     if query.dtype == torch.float32 and value.stride(-1) != 1:
         return False  # the fp32 kernel reads V head_dim-contiguous
     per_16_bytes = 16 // query.element_size()
+    shape = query.shape
     for tensor in (query, key, value):
         if tensor.data_ptr() % 16:
             return False
-        if any(stride % per_16_bytes for stride in _strides(tensor) if stride != 1):
-            return False
+        for size, stride in zip(shape, tensor.stride()):
+            if stride % per_16_bytes and stride != 1 and size != 1:
+                return False
     if not hip_streaming_dh64_causal_attention_available():
         return False
     return is_gfx950(query.device)
@@ -261,7 +275,22 @@ def prevalidated_hip_streaming_dh64_causal_attention_bsd(
     """Run the kernel after immutable execution-plan validation."""
 
     _validate_launch_config(block_m, block_n, num_warps, num_stages)
-    resolved_scale = 1.0 / math.sqrt(_HEAD_DIM) if scale is None else float(scale)
+    return _run(query, key, value, scale, block_m, block_n, num_warps, num_stages)
+
+
+def _run(
+    query: torch.Tensor,
+    key: torch.Tensor,
+    value: torch.Tensor,
+    scale: float | None,
+    block_m: int,
+    block_n: int,
+    num_warps: int,
+    num_stages: int,
+) -> tuple[torch.Tensor, str]:
+    """The launch, its parameters validated."""
+
+    resolved_scale = _DEFAULT_SCALE if scale is None else float(scale)
     try:
         if torch.compiler.is_compiling():
             output = _streaming_dh64_causal_attention_bsd_op(
@@ -307,16 +336,7 @@ def hip_streaming_dh64_causal_attention_bsd(
         raise RuntimeError(
             "HIP streaming attention is ineligible for the requested inputs"
         )
-    return prevalidated_hip_streaming_dh64_causal_attention_bsd(
-        query,
-        key,
-        value,
-        scale=scale,
-        block_m=block_m,
-        block_n=block_n,
-        num_warps=num_warps,
-        num_stages=num_stages,
-    )
+    return _run(query, key, value, scale, block_m, block_n, num_warps, num_stages)
 
 
 __all__ = [

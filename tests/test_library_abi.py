@@ -316,3 +316,27 @@ def test_mlp_residual_norm_entry_validates_before_launch():
     assert call(x=None) == _library.SAH_ERR_INVALID_ARGUMENT
     assert call(x=ctypes.c_void_p(4096 + 8)) == _library.SAH_ERR_INVALID_ARGUMENT
     assert call(b1=ctypes.c_void_p(4096 + 4)) == _library.SAH_ERR_INVALID_ARGUMENT
+
+
+@pytest.mark.parametrize("launch", [(256, 256, 64, 8), (128, 256, 64, 8), (256, 128, 64, 8), (256, 256, 32, 8),
+                                    (256, 256, 64, 4), (0, 0, 0, 0), (-256, 256, 64, 8)])
+def test_python_launch_tables_agree_with_the_library(launch):
+    """The wrappers' own tables, which they read instead of asking per call."""
+
+    from solution.kernels.boundary.hip_linear_residual_norm import launch_config_is_valid as boundary
+    from solution.kernels.ffn.hip_linear_gelu import launch_config_is_valid as linear
+    from solution.kernels.projection.hip_qkv_layout import launch_config_is_valid as qkv
+
+    library = _library.load_library()
+    assert qkv(*launch) == bool(library.sah_qkv_launch_supported(*launch))
+    for stages in (1, 2, 3):
+        assert linear(*launch, stages) == bool(
+            library.sah_linear_launch_supported(*launch, stages)
+        )
+    for width in (256, 512, 1024, 2048):
+        for rows in (launch[2], 32, 64, 128, 256):
+            for warps in (4, 8):
+                assert boundary(width, rows, warps) == bool(
+                    library.sah_linear_residual_norm_launch_supported(width, rows, warps)
+                )
+    assert not linear(256.0, 256, 64, 8, 2) and not qkv(256.0, 256, 64, 8) and not boundary(512.0, 128, 8)
