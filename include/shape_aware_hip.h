@@ -239,10 +239,11 @@ int sah_linear(
     sah_stream_t stream);
 
 /*
- * fp32 Linear y = x weight^T + bias (the projections of small fp32 models:
- * nn.Linear of the reference's portable path, solution/transformer.py:291-353).
- * fp32 accumulation on the fp32 matrix cores, four ranges of K
- * summed in ascending order.  x: [rows, in_features] with row stride x_row_stride;
+ * fp32 Linear y = act(x weight^T + bias) (the projections of small fp32 models:
+ * nn.Linear and F.gelu of the reference's portable path,
+ * solution/transformer.py:291-353).  activation is an enum of sah_linear's
+ * (exact GELU through erff).  fp32 accumulation on the fp32 matrix cores, four
+ * or eight ranges of K summed in ascending order.  x: [rows, in_features] with row stride x_row_stride;
  * weight: [out_features, in_features] contiguous; bias: [out_features] or
  * NULL; y: [rows, out_features] with row stride y_row_stride, overlapping no
  * input.  in_features a multiple of 128, out_features of 32; row strides
@@ -251,7 +252,7 @@ int sah_linear(
 int sah_linear_f32(
     const float* x, const float* weight, const float* bias, float* y,
     int64_t rows, int64_t in_features, int64_t out_features,
-    int64_t x_row_stride, int64_t y_row_stride, sah_stream_t stream);
+    int64_t x_row_stride, int64_t y_row_stride, int activation, sah_stream_t stream);
 
 /* 1 if sah_linear implements this launch, else 0 (mirrors the reference's
  * _launch_config_is_valid, solution/kernels/ffn/triton_linear_exact_gelu.py:29-45). */

@@ -1,4 +1,4 @@
-// fp32 Linear y = x W^T + b for few rows, on the fp32 matrix cores (gfx950).
+// fp32 Linear y = act(x W^T + b) for few rows, on the fp32 matrix cores (gfx950).
 //
 // For the projections of small fp32 models (a few hundred rows, K and N of a
 // few hundred), where a library GEMM of large tiles leaves most CUs idle
@@ -11,23 +11,44 @@
 //  * Operands go straight to registers, 16 bytes a lane (lane half h of slice
 //    u holds K 8 u + 4 h .. + 3 of its row on both sides), 32 of K ahead of
 //    their use.  Neighbouring tiles share x and W through L2.
-// The sums of the quarters are added in ascending order, then the bias.
-// Measured (us, GPU time, library -> this): 256 x 256 -> 256 63 -> 4.8, 256 x
-// 256 -> 1024 5.7 -> 5.1, 100 x 128 -> 128 11.4 -> 3.9; with more tiles than
-// CUs or a longer K the library is faster (512 x 256 -> 768 5.8 against 7.8,
-// 256 x 1024 -> 256 5.8 against 10.0: the 32-byte row segments of the loads).
+//  * A longer K takes 16 x 16 tiles and eight waves (v_mfma_f32_16x16x4):
+//    four times the workgroups, and up to K 1024 a wave's loads are one batch.
+// The sums of the ranges are added in ascending order, then the bias, then
+// GELU (its pass over memory and its launch go: 256 x 256 -> 1024 with it 8.2
+// us by library and elementwise kernel, 5.3 here).
+// Measured (us, GPU time, library -> this): 256 x 256 -> 256 63 -> 4.7, 256 x
+// 256 -> 1024 5.6 -> 4.9, 100 x 128 -> 128 11.4 -> 3.8, 256 x 512 -> 256 117
+// -> 5.9, 256 x 1024 -> 256 5.8 -> 6.0; with more tiles than CUs or a longer K
+// the library is faster (512 x 256 -> 768 5.8 against 7.8, 256 x 2048 -> 256
+// 7.1 against 10.4: the short row segments of the loads).
 #include "sah_common.hpp"
 
 namespace sah {
 namespace {
 
 constexpr int kTile = 32;
+constexpr int kSmallTile = 16;
+constexpr int kSmallSplit = 8;
+constexpr int kSmallAhead = 8;  // slices of 16 loaded ahead (128 of K: all of a wave's up to K 1024)
+// The small tiles serve a longer K, while they fit one round of the CUs (us,
+// 32 x 32 / 16 x 16): 256 x 256 -> 256 4.7 / 5.7, 100 x 384 -> 384 5.5 / 5.7,
+// 256 x 512 -> 256 6.4 / 5.9, 256 x 1024 -> 256 9.8 / 6.0.
+constexpr int kMaxWide = 384;
+constexpr int kMaxTiles = 256;
 constexpr int kSplit = 4;    // waves sharing a tile's K
 constexpr int kAhead = 4;    // slices of 8 loaded ahead (32 of K)
 
 __device__ __forceinline__ f32x16 mfma32x2(float a, float b, f32x16 c) {
   return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
 }
+
+__device__ __forceinline__ f32x4 mfma16x4(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+// v Phi(v) by the device library's erff, as the framework's own fp32 GELU has
+// it (16-bit outputs take the cheaper gelu_exact).
+__device__ __forceinline__ float gelu_f32(float v) { return 0.5f * v * (1.0f + erff(v * 7.071067812e-01f)); }
 
 struct LinearF32Params {
   const float* x;
@@ -38,6 +59,7 @@ struct LinearF32Params {
   int n, k;
 };
 
+template <bool GELU>
 __global__ __launch_bounds__(kSplit * 64) void linear_f32_kernel(LinearF32Params p) {
   __shared__ __attribute__((aligned(16))) float part[kSplit][kTile][kTile + 4];
   const int lane = threadIdx.x & 63;
@@ -95,6 +117,77 @@ __global__ __launch_bounds__(kSplit * 64) void linear_f32_kernel(LinearF32Params
 #pragma unroll
   for (int s = 1; s < kSplit; ++s) sum += *reinterpret_cast<const f32x4*>(&part[s][out_row][col]);
   if (p.bias != nullptr) sum += *reinterpret_cast<const f32x4*>(p.bias + n0 + col);
+  if (GELU)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum[i] = gelu_f32(sum[i]);
+  *reinterpret_cast<f32x4*>(p.y + (m0 + out_row) * p.y_ld + n0 + col) = sum;
+}
+
+// The same on 16 x 16 tiles, eight waves an eighth of K each: for so few
+// outputs that these tiles still fit one round of the CUs.
+template <bool GELU>
+__global__ __launch_bounds__(kSmallSplit * 64) void linear_f32_small_kernel(LinearF32Params p) {
+  __shared__ __attribute__((aligned(16))) float part[kSmallSplit][kSmallTile][kSmallTile + 4];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l16 = lane & 15;
+  const int quarter = lane >> 4;
+  const unsigned tiles_n = (unsigned)(p.n / kSmallTile);
+  const unsigned tile_m = blockIdx.x / tiles_n;
+  const int n0 = (int)(blockIdx.x - tile_m * tiles_n) * kSmallTile;
+  const int64_t m0 = (int64_t)tile_m * kSmallTile;
+  const int range = p.k / kSmallSplit;  // a multiple of 16
+  const int slices = range / 16;
+  // rows past the end read the last row; they are not stored
+  const int64_t row = m0 + l16 < p.rows ? m0 + l16 : p.rows - 1;
+  // slice u: lane quarter q holds K 16 u + 4 q .. + 3 of its row on both sides
+  const float* x = p.x + row * p.x_ld + wave * range + 4 * quarter;
+  const float* w = p.w + (int64_t)(n0 + l16) * p.k + wave * range + 4 * quarter;
+
+  f32x4 xa[kSmallAhead], wa[kSmallAhead];
+#pragma unroll
+  for (int u = 0; u < kSmallAhead; ++u) {
+    const int at = 16 * (u < slices ? u : slices - 1);
+    xa[u] = *reinterpret_cast<const f32x4*>(x + at);
+    wa[u] = *reinterpret_cast<const f32x4*>(w + at);
+  }
+  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  for (int s = 0; s < slices; s += kSmallAhead) {
+    // the next slices (past the end the last one again: in bounds, not used)
+    f32x4 xb[kSmallAhead] = {}, wb[kSmallAhead] = {};
+    if (s + kSmallAhead < slices)
+#pragma unroll
+      for (int u = 0; u < kSmallAhead; ++u) {
+        const int next = s + kSmallAhead + u;
+        const int at = 16 * (next < slices ? next : slices - 1);
+        xb[u] = *reinterpret_cast<const f32x4*>(x + at);
+        wb[u] = *reinterpret_cast<const f32x4*>(w + at);
+      }
+#pragma unroll
+    for (int u = 0; u < kSmallAhead; ++u)
+      if (s + u < slices)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc = mfma16x4(wa[u][i], xa[u][i], acc);
+#pragma unroll
+    for (int u = 0; u < kSmallAhead; ++u) {
+      xa[u] = xb[u];
+      wa[u] = wb[u];
+    }
+  }
+  // acc[r]: column 4 quarter + r of row l16
+  *reinterpret_cast<f32x4*>(&part[wave][l16][4 * quarter]) = acc;
+  __syncthreads();
+  if (wave != 0) return;
+  const int out_row = lane >> 2;
+  const int col = (lane & 3) * 4;
+  if (m0 + out_row >= p.rows) return;
+  f32x4 sum = *reinterpret_cast<const f32x4*>(&part[0][out_row][col]);
+#pragma unroll
+  for (int s = 1; s < kSmallSplit; ++s) sum += *reinterpret_cast<const f32x4*>(&part[s][out_row][col]);
+  if (p.bias != nullptr) sum += *reinterpret_cast<const f32x4*>(p.bias + n0 + col);
+  if (GELU)
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum[i] = gelu_f32(sum[i]);
   *reinterpret_cast<f32x4*>(p.y + (m0 + out_row) * p.y_ld + n0 + col) = sum;
 }
 
@@ -105,7 +198,9 @@ using namespace sah;
 
 extern "C" int sah_linear_f32(const float* x, const float* weight, const float* bias, float* y, int64_t rows,
                               int64_t in_features, int64_t out_features, int64_t x_row_stride,
-                              int64_t y_row_stride, sah_stream_t stream) {
+                              int64_t y_row_stride, int activation, sah_stream_t stream) {
+  if (activation != SAH_ACTIVATION_NONE && activation != SAH_ACTIVATION_GELU_EXACT)
+    return fail(SAH_ERR_INVALID_ARGUMENT, "sah_linear_f32: unknown activation %d", activation);
   if (rows < 0 || in_features <= 0 || out_features <= 0)
     return fail(SAH_ERR_INVALID_ARGUMENT, "sah_linear_f32: bad sizes rows=%lld in=%lld out=%lld", (long long)rows,
                 (long long)in_features, (long long)out_features);
@@ -136,7 +231,12 @@ extern "C" int sah_linear_f32(const float* x, const float* weight, const float* 
   p.y_ld = y_row_stride;
   p.n = (int)out_features;
   p.k = (int)in_features;
-  hipLaunchKernelGGL(linear_f32_kernel, dim3((unsigned)tiles), dim3(kSplit * 64), 0,
-                     reinterpret_cast<hipStream_t>(stream), p);
+  const bool gelu = activation == SAH_ACTIVATION_GELU_EXACT;
+  const int64_t small_tiles = ceil_div(rows, kSmallTile) * (out_features / kSmallTile);
+  const bool small = in_features > kMaxWide && small_tiles <= kMaxTiles;
+  auto* kernel = small ? (gelu ? linear_f32_small_kernel<true> : linear_f32_small_kernel<false>)
+                       : (gelu ? linear_f32_kernel<true> : linear_f32_kernel<false>);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)(small ? small_tiles : tiles)),
+                     dim3(64 * (small ? kSmallSplit : kSplit)), 0, reinterpret_cast<hipStream_t>(stream), p);
   return check_hip(hipGetLastError(), "fp32 linear kernel launch");
 }

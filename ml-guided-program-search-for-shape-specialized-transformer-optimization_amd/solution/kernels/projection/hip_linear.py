@@ -13,23 +13,29 @@ import torch
 from torch import nn
 
 from ..hip._library import (
+    SAH_ACTIVATION_GELU_EXACT,
+    SAH_ACTIVATION_NONE,
     check_status,
     is_gfx950,
     load_library,
     stream_handle,
 )
 
-# The 32 x 32 tiles that one round of the 256 CUs takes, and the K whose row
-# segments the loads read well (GPU time in us, library / this kernel):
-#   256 x 256 -> 256     63 / 4.8     512 x 256 -> 768     5.8 /  7.8
-#   256 x 256 -> 1024   5.7 / 5.1    1024 x 256 -> 1024    8.0 / 13.8
-#   100 x 128 -> 128   11.4 / 3.9     256 x 1024 -> 256    5.8 / 10.0
-# A call also costs the host about half of F.linear's.  (The 16-bit tile
-# kernels were tried here too: at 16384 x 512 -> 1536 and 512 -> 512 they are
-# 4-9% faster than the library alone, but the forward of that stack measured
-# the same, 835 us.)
+# One round of the 256 CUs in 32 x 32 tiles, or for a longer K in 16 x 16
+# tiles (GPU time in us, library / this kernel):
+#   256 x 256 -> 256     63 / 4.7     512 x 256 -> 768     5.8 /  7.8
+#   256 x 256 -> 1024   5.6 / 4.9    1024 x 256 -> 1024    8.0 / 13.8
+#   100 x 128 -> 128   11.4 / 3.8
+#   256 x 512 -> 256    117 / 5.9     256 x 2048 -> 256    7.1 / 10.4
+#   256 x 1024 -> 256   5.8 / 6.0
+# A call also costs the host about half of F.linear's (10 us less), which is
+# what bounds a forward of these sizes; with GELU the elementwise launch goes
+# too (256 x 256 -> 1024 8.2 / 5.3).  (The 16-bit tile kernels were tried here
+# too: at 16384 x 512 -> 1536 and 512 -> 512 they are 4-9% faster than the
+# library alone, but the forward of that stack measured the same, 835 us.)
 _MAX_TILES = 256
 _MAX_IN = 384
+_MAX_IN_SMALL_TILES = 1024
 
 
 def _serves(rows: int, in_features: int, out_features: int, dtype: torch.dtype) -> bool:
@@ -37,10 +43,15 @@ def _serves(rows: int, in_features: int, out_features: int, dtype: torch.dtype) 
 
     return (
         dtype == torch.float32
-        and in_features <= _MAX_IN
+        and in_features <= _MAX_IN_SMALL_TILES
         and in_features % 128 == 0
         and out_features % 32 == 0
-        and (rows + 31) // 32 * (out_features // 32) <= _MAX_TILES
+        and (
+            (rows + 31) // 32 * (out_features // 32)
+            if in_features <= _MAX_IN
+            else (rows + 15) // 16 * (out_features // 16)
+        )
+        <= _MAX_TILES
     )
 
 
@@ -68,9 +79,10 @@ def _is_plain(module: nn.Linear, value: torch.Tensor) -> bool:
     )
 
 
-def project(module: nn.Linear, value: torch.Tensor) -> torch.Tensor | None:
-    """``module(value)`` on the gfx950 kernel, or None where they do not
-    serve the call (size, type, layout, or a call that something observes)."""
+def project(module: nn.Linear, value: torch.Tensor, *, gelu: bool = False) -> torch.Tensor | None:
+    """``module(value)``, with ``gelu`` the exact GELU of it, on the gfx950
+    kernel, or None where it does not serve the call (size, type, layout, or a
+    call that something observes)."""
 
     weight, bias = module.weight, module.bias
     dtype = value.dtype
@@ -100,6 +112,7 @@ def project(module: nn.Linear, value: torch.Tensor) -> torch.Tensor | None:
         out_features,
         in_features,
         out_features,
+        SAH_ACTIVATION_GELU_EXACT if gelu else SAH_ACTIVATION_NONE,
         stream_handle(value.device),
     )
     check_status(status, "sah_linear_f32")

@@ -553,13 +553,20 @@ class _TransformerBlock(nn.Module):
                 marker, expected_marker=HIP_EXACT_GELU_BACKEND, planned_backend=plan.ffn_backend.value
             )
         else:
-            projected = self.ffn_in.forward_backend(
-                normalized, plan.ffn_input_projection_backend, hip=plan.uses_hip_attention
-            )
-            input_compute_dtype = _dtype_name(projected.dtype)
-            if plan.ffn_activation_output_dtype == "float32":
-                projected = projected.float()
-            hidden = F.gelu(projected, approximate="none")
+            hidden = None
+            if plan.uses_hip_attention and plan.ffn_input_projection_backend is ProjectionBackend.INPUT_DTYPE:
+                from .kernels.projection.hip_linear import project as hip_project
+
+                # a small fp32 projection and its GELU as one launch
+                hidden = hip_project(self.ffn_in, normalized, gelu=True)
+            if hidden is not None:
+                input_compute_dtype = _dtype_name(hidden.dtype)
+            else:
+                projected = self.ffn_in.forward_backend(normalized, plan.ffn_input_projection_backend)
+                input_compute_dtype = _dtype_name(projected.dtype)
+                if plan.ffn_activation_output_dtype == "float32":
+                    projected = projected.float()
+                hidden = F.gelu(projected, approximate="none")
         update = (
             self.ffn_out.forward_backend(
                 hidden, plan.ffn_output_projection_backend, hip=plan.uses_hip_attention

@@ -199,11 +199,13 @@ def test_rows_beyond_the_tile_kernels_offsets(gpu_device):
 
 
 @pytest.mark.parametrize("rows", [1, 31, 33, 256])
-@pytest.mark.parametrize("k,n", [(128, 32), (256, 256), (384, 96), (1024, 64)])
+@pytest.mark.parametrize("k,n", [(128, 32), (256, 256), (384, 96), (512, 32), (1024, 64), (1152, 64), (512, 1024)])
 def test_fp32_linear_at_its_edges(gpu_device, rows, k, n):
-    """sah_linear_f32 about its 32 x 32 tiles and 32-wide load steps, with
-    padded rows on both sides, against float64: k products and sums in fp32,
-    (k + 4) 2^-24 of sum |x| |w| + |b|."""
+    """sah_linear_f32 about its 32 x 32 and 16 x 16 tiles and their load steps,
+    with padded rows on both sides, against float64: k products and sums in
+    fp32, (k + 4) 2^-24 of sum |x| |w| + |b|.  GELU: its slope (at most 1.13)
+    times that, and 5 2^-24 |v| for 0.5 v (1 + erff(v / sqrt 2)) (erff to 2
+    ulp, its argument and the sum to one rounding each, two products)."""
 
     from solution.kernels.hip import _library
 
@@ -213,20 +215,24 @@ def test_fp32_linear_at_its_edges(gpu_device, rows, k, n):
     xs[:, :k] = torch.randn(rows, k, generator=g)
     w, b = torch.randn(n, k, generator=g).to(gpu_device), torch.randn(n, generator=g).to(gpu_device)
     xs = xs.to(gpu_device)
-    for bias in (b, None):
+    for bias, act in ((b, 0), (None, 0), (b, 1)):
         y = torch.full((rows + 2, ldy), -7.0, device=gpu_device)
         status = _library.load_library().sah_linear_f32(
             xs.data_ptr(), w.data_ptr(), None if bias is None else bias.data_ptr(), y.data_ptr(), rows, k, n, ldx,
-            ldy, _library.stream_handle(gpu_device),
+            ldy, act, _library.stream_handle(gpu_device),
         )
         _library.check_status(status, "sah_linear_f32")
         torch.cuda.synchronize()
         x = xs[:, :k].double()
         expected = F.linear(x, w.double(), None if bias is None else bias.double())
         size = F.linear(x.abs(), w.double().abs(), None if bias is None else bias.double().abs())
+        bound = (k + 4) * 2.0**-24 * size
+        if act:
+            bound = 1.13 * bound + 5 * 2.0**-24 * expected.abs()
+            expected = F.gelu(expected)
         error = (y[:rows, :n].double() - expected).abs()
-        print(f"fp32 linear {rows}x{k}->{n}: max err {float(error.max()):.3g}", flush=True)
-        assert bool((error <= (k + 4) * 2.0**-24 * size).all())
+        print(f"fp32 linear {rows}x{k}->{n} act {act}: max err {float(error.max()):.3g}", flush=True)
+        assert bool((error <= bound).all())
         assert bool((y[:rows, n:] == -7.0).all()) and bool((y[rows:] == -7.0).all())
 
 
@@ -246,6 +252,9 @@ def test_model_projection_takes_what_it_serves(gpu_device):
         size = F.linear(value.double().abs(), linear.weight.double().abs(), linear.bias.double().abs())
         bound = (k + 4) * 2.0**-24 * size
         assert out.shape == (1, rows, n) and bool(((out.double() - exact).abs() <= bound).all())
+        hidden = project(linear, value, gelu=True)
+        bound = 1.13 * bound + 5 * 2.0**-24 * exact.abs()
+        assert bool(((hidden.double() - F.gelu(exact)).abs() <= bound).all())
         assert project(linear, torch.randn(1, rows, k + 8, device=gpu_device, dtype=dtype)[..., :k]) is None
         assert project(linear, value.cpu()) is None
         with torch.autocast("cuda", dtype=torch.float16):

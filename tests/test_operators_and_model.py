@@ -154,7 +154,8 @@ def test_model_projection_rule():
 
     f32 = torch.float32
     assert _serves(256, 256, 1024, f32) and _serves(1, 384, 32, f32) and _serves(8192, 128, 32, f32)
-    for sizes in [(257, 256, 1024), (256, 512, 256), (256, 192, 256), (256, 256, 200)]:
+    assert _serves(256, 1024, 256, f32) and _serves(16, 512, 4096, f32)
+    for sizes in [(257, 256, 1024), (256, 192, 256), (256, 256, 200), (257, 1024, 256), (16, 1152, 256)]:
         assert not _serves(*sizes, f32), sizes
     for dtype in (torch.float64, torch.bfloat16, torch.float16):
         assert not _serves(64, 256, 256, dtype)
