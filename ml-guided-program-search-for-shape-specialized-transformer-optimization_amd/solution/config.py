@@ -156,8 +156,8 @@ HIP_RESIDUAL_NORM_BACKENDS = frozenset(
         ResidualNormBackend.HIP_LINEAR_FUSED,
     }
 )
-# Backends that fuse the branch's output projection into the residual
-# boundary (the update never reaches HBM).
+# Backends that take the branch's output projection into the residual
+# boundary, as one operator.
 LINEAR_BOUNDARY_RESIDUAL_NORM_BACKENDS = frozenset(
     {ResidualNormBackend.TRITON_LINEAR_MIXED, ResidualNormBackend.HIP_LINEAR_FUSED}
 )
