@@ -372,11 +372,11 @@ int launch_linear_tiles(LinearParams prm, hipStream_t stream) {
   // ((TM + TN) rows of 128 bytes at about 60 GB/s) or multiplies; two 64 x 64
   // workgroups share a CU.  Measured (bf16 Linear, us), 64 x 64, 128 x 128,
   // 128 x 256 and 256 x 256:
-  //   64 x 4096 -> 1024     19.9   35.8   43.8   68.0
-  //   800 x 2048 -> 512     11.8   19.9   25.1   38.4
-  //   777 x 1024 -> 4096    16.3   13.4   16.5   24.3
-  //   2000 x 1024 -> 3072   25.5   24.0   18.8   25.9
-  //   6000 x 1024 -> 4096   93.7   73.5   57.5   55.6
+  //   64 x 4096 -> 1024     19.7   37.4   43.8   68.0
+  //   800 x 2048 -> 512     12.0   20.7   25.1   38.4
+  //   777 x 1024 -> 4096    17.1   13.1   16.5   24.3
+  //   2000 x 1024 -> 3072   24.2   23.7   18.8   25.9
+  //   6000 x 1024 -> 4096   89.1   72.0   57.5   55.6
   //   16384 x 2048 -> 512            42     36     43
   //   20002 x 1024 -> 3072          170    144    118
   const int64_t cus = compute_units();
