@@ -95,7 +95,10 @@ __global__ __launch_bounds__(kSplit * 64, 2) void attn_fwd_f32_kernel(AttnF32Par
   f32x16 o0, o1;
 #pragma unroll
   for (int r = 0; r < 16; ++r) o0[r] = o1[r] = 0.0f;
-  float m_run = -INFINITY, l_run = 0.0f;  // of this wave's keys; l_run of this half's
+  // Of this wave's keys; l_run of this half's.  The maximum starts at the
+  // lowest shift instead of -inf: keys that all score -inf (or too low for the
+  // shift) then weigh exp2(-inf) = 0, and nothing forms -inf + inf.
+  float m_run = p.floor, l_run = 0.0f;
   auto load_k = [&](const float* row) {
 #pragma unroll
     for (int u = 0; u < 8; ++u) kf[u] = *reinterpret_cast<const f32x4*>(row + 8 * u);
@@ -220,8 +223,8 @@ __global__ __launch_bounds__(kSplit * 64, 2) void attn_fwd_f32_kernel(AttnF32Par
   }
   __syncthreads();
 
-  // Merge: eight threads per query, 8 dims each.  A wave without a block has
-  // maximum -inf, sum 0 and output 0; wave 0 always has one.
+  // Merge: eight threads per query, 8 dims each.  A wave without a block, or
+  // with no key above -inf, has the lowest shift, sum 0 and output 0.
   const int row = tid >> 3;
   const int d0 = (tid & 7) * 8;
   if (qt * kQ + row >= S) return;

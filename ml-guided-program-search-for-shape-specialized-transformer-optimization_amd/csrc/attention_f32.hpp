@@ -18,7 +18,8 @@ struct AttnF32Params {
   int64_t o_sb, o_ss;
   int seq_len;
   int heads;
-  float c;  // |scale| log2(e), > 0
+  float c;      // |scale| log2(e), > 0
+  float floor;  // the lowest shift: the most negative float whose product with c is finite
   uint32_t q_and, q_xor;  // the sign of the scale (or a zero scale), on Q
 };
 

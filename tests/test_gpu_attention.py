@@ -667,3 +667,41 @@ def test_fp32_attention_block_edges_against_float64(gpu_device, batch, heads, se
     error = float((output.double() - expected).abs().max())
     print(f"  max error {error:.3g}, bound {bound:.3g}", flush=True)
     assert error <= bound
+
+
+@pytest.mark.parametrize("seq", [200, 261])
+@pytest.mark.parametrize("blocks", [(0,), (1,), (2, 3), (1, 2, 3), (0, 1, 2), (4, 5)])
+@pytest.mark.parametrize("low,scale", [(float("-inf"), 0.125), (float("-inf"), 4.0), (-1e38, 8.0)])
+def test_fp32_attention_with_key_blocks_below_every_shift(gpu_device, seq, blocks, low, scale):
+    """Whole 32-key blocks that score -inf (or so low that scale times the
+    score overflows) weigh nothing: their wave's share of the keys must not
+    make the others' NaN.  Against float64, for every query that sees another
+    key; a query that sees only -inf scores is NaN, as in softmax.
+
+    Bound: that of test_fp32_attention_block_edges_against_float64, the low
+    component left out of sum |q k| (it decides only which keys count)."""
+
+    heads = 2
+    print(f"fp32 low blocks {blocks} seq {seq} low {low} scale {scale}", flush=True)
+    q, k, v = (t.to(gpu_device) for t in _inputs(1, heads, seq, dtype=torch.float32, seed=seq))
+    q[..., 0] = 1.0
+    magnitude = q.double().abs() @ k.double().abs().transpose(-1, -2).contiguous()
+    hidden = torch.zeros(seq, dtype=torch.bool, device=gpu_device)
+    for block in blocks:
+        hidden[32 * block : 32 * block + 32] = True
+    k[..., 0].masked_fill_(hidden, low)
+    module = _attention_module()
+    with torch.inference_mode():
+        output, _ = module.hip_streaming_dh64_causal_attention_bsd(q, k, v, scale=scale)
+    torch.cuda.synchronize(gpu_device)
+    scores = q.double() @ k.double().transpose(-1, -2).contiguous() * scale
+    future = torch.ones(seq, seq, dtype=torch.bool, device=gpu_device).triu(1)
+    expected = _to_bsd(torch.softmax(scores.masked_fill(future, float("-inf")), dim=-1) @ v.double())
+    sees = (~hidden).cumsum(0) > 0
+    d = 64 * 2.0**-24 * float(magnitude.max()) * scale
+    bound = float(v.abs().max()) * (2.1 * d + (seq + 8) * 2.0**-24)
+    error = float((output.double() - expected)[:, sees].abs().max())
+    print(f"  max error {error:.3g}, bound {bound:.3g}", flush=True)
+    assert error <= bound  # false for NaN
+    if math.isinf(low):
+        assert bool(torch.isnan(output[:, ~sees]).all())
