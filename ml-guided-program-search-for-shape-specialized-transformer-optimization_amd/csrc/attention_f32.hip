@@ -98,7 +98,7 @@ __global__ __launch_bounds__(kSplit * 64, 2) void attn_fwd_f32_kernel(AttnF32Par
   // Of this wave's keys; l_run of this half's.  The maximum starts at the
   // lowest shift instead of -inf: keys that all score -inf (or too low for the
   // shift) then weigh exp2(-inf) = 0, and nothing forms -inf + inf.
-  float m_run = p.floor, l_run = 0.0f;
+  float m_run = p.floor, mc_run = p.floor * c, l_run = 0.0f;
   auto load_k = [&](const float* row) {
 #pragma unroll
     for (int u = 0; u < 8; ++u) kf[u] = *reinterpret_cast<const f32x4*>(row + 8 * u);
@@ -113,6 +113,17 @@ __global__ __launch_bounds__(kSplit * 64, 2) void attn_fwd_f32_kernel(AttnF32Par
       for (int i = 0; i < 4; ++i) s = mfma32x2(kf[u][i], q[u][i], s);
     return s;
   };
+  // The shift c m as one rounded number, the same for P, the rescaling and the
+  // merge (the assembly keeps it from being formed again inside an fma there):
+  // its rounding then cancels, where exp2(c (m_run - m_new)) beside it is off by
+  // half an ulp of c m (error against float64, relative to the 64-key-tile
+  // kernel's, over S 31-2500: 0.98-1.02 -> 0.97-1.01; with scores about 77000
+  // 1.4e-4 -> 2.4e-7).
+  auto shift = [&](float m) {
+    float mc = m * c;
+    asm("" : "+v"(mc));
+    return mc;
+  };
   // P = exp2(c (s - m)) in place, the row sums and the outputs rescaled.
   auto softmax = [&](f32x16& s) {
     float mx = s[0];
@@ -120,9 +131,10 @@ __global__ __launch_bounds__(kSplit * 64, 2) void attn_fwd_f32_kernel(AttnF32Par
     for (int r = 1; r < 16; ++r) mx = fmaxf(mx, s[r]);
     mx = fmaxf(mx, __shfl_xor(mx, 32));
     const float m_new = fmaxf(m_run, mx);
-    const float alpha = __builtin_amdgcn_exp2f((m_run - m_new) * c);
+    const float mc = shift(m_new);
+    const float alpha = __builtin_amdgcn_exp2f(mc_run - mc);
     m_run = m_new;
-    const float mc = m_new * c;
+    mc_run = mc;
     float sum = 0.0f;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
@@ -160,9 +172,10 @@ __global__ __launch_bounds__(kSplit * 64, 2) void attn_fwd_f32_kernel(AttnF32Par
         if (n == 7) other = __shfl_xor(mx, 32);
         if (n == 13) {
           const float m_new = fmaxf(m_run, fmaxf(mx, other));
-          alpha = __builtin_amdgcn_exp2f((m_run - m_new) * c);
+          mc = shift(m_new);
+          alpha = __builtin_amdgcn_exp2f(mc_run - mc);
           m_run = m_new;
-          mc = m_new * c;
+          mc_run = mc;
         }
         if (n >= 14 && n < 30) {
           const int r = n - 14;
@@ -218,7 +231,7 @@ __global__ __launch_bounds__(kSplit * 64, 2) void attn_fwd_f32_kernel(AttnF32Par
   }
   l_run += __shfl_xor(l_run, 32);
   if (half == 0) {
-    m_lds[wave][l32] = m_run;
+    m_lds[wave][l32] = mc_run;
     l_lds[wave][l32] = l_run;
   }
   __syncthreads();
@@ -228,14 +241,14 @@ __global__ __launch_bounds__(kSplit * 64, 2) void attn_fwd_f32_kernel(AttnF32Par
   const int row = tid >> 3;
   const int d0 = (tid & 7) * 8;
   if (qt * kQ + row >= S) return;
-  float m_all = m_lds[0][row];
+  float m_all = m_lds[0][row];  // shifts c m
 #pragma unroll
   for (int w = 1; w < kSplit; ++w) m_all = fmaxf(m_all, m_lds[w][row]);
   float l_all = 0.0f;
   f32x4 lo = {0.0f, 0.0f, 0.0f, 0.0f}, hi = lo;
 #pragma unroll
   for (int w = 0; w < kSplit; ++w) {
-    const float scale = __builtin_amdgcn_exp2f((m_lds[w][row] - m_all) * c);
+    const float scale = __builtin_amdgcn_exp2f(m_lds[w][row] - m_all);
     l_all = fmaf(l_lds[w][row], scale, l_all);
     const f32x4 a = *reinterpret_cast<const f32x4*>(&o_lds[w][row][d0]);
     const f32x4 d = *reinterpret_cast<const f32x4*>(&o_lds[w][row][d0 + 4]);

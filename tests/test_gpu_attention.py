@@ -705,3 +705,37 @@ def test_fp32_attention_with_key_blocks_below_every_shift(gpu_device, seq, block
     assert error <= bound  # false for NaN
     if math.isinf(low):
         assert bool(torch.isnan(output[:, ~sees]).all())
+
+
+@pytest.mark.parametrize("seq", [64, 333, 1000])
+def test_fp32_attention_with_a_large_common_score(gpu_device, seq):
+    """Scores of about 77 000 that differ by a few tens, all exact integers:
+    only differences count in softmax, so the rounding of the common part must
+    not show between the key blocks.  Against float64.
+
+    Bound on a weight's relative error, with E the largest exponent |c (s - m)|:
+    c is one rounded product (2^-23 E ln 2), a key's exponent one rounding and
+    each rescaling (at most one per block of its wave, seq / 128 + 1, and the
+    merge) another (2^-24 E ln 2 each) with its exp2 (2^-23 each); outputs move
+    by twice that of max |v|, and sums add (seq + 8) 2^-24 max |v|."""
+
+    heads = 2
+    print(f"fp32 common score seq {seq}", flush=True)
+    g = torch.Generator().manual_seed(seq)
+    q, k = (torch.randint(-1, 2, (1, heads, seq, 64), generator=g).float().to(gpu_device) for _ in range(2))
+    v = torch.randn(1, heads, seq, 64, generator=g).to(gpu_device)
+    q[..., 0], k[..., 0] = 300.0, 256.0
+    module = _attention_module()
+    with torch.inference_mode():
+        output, _ = module.hip_streaming_dh64_causal_attention_bsd(q, k, v)
+    torch.cuda.synchronize(gpu_device)
+    scores = q.double() @ k.double().transpose(-1, -2).contiguous() / 8
+    future = torch.ones(seq, seq, dtype=torch.bool, device=gpu_device).triu(1)
+    expected = _to_bsd(torch.softmax(scores.masked_fill(future, float("-inf")), dim=-1) @ v.double())
+    exponent = math.log2(math.e) * float(scores.max() - scores.min())
+    rescalings = seq // 128 + 3
+    weight = 2.0**-24 * ((3 + rescalings) * exponent + 2 * (1 + rescalings))
+    bound = float(v.abs().max()) * (2 * weight + (seq + 8) * 2.0**-24)
+    error = float((output.double() - expected).abs().max())
+    print(f"  max error {error:.3g}, bound {bound:.3g}", flush=True)
+    assert error <= bound
