@@ -163,7 +163,9 @@ int sah_causal_attention_launch_supported(int block_m, int block_n, int num_warp
  *   residual   = round_to(value_dtype, value + update)
  *   normalized = round_to(normalized_dtype, norm(residual) * weight + bias)
  * Statistics are fp32, computed in one pass over HBM (per-lane Welford states
- * merged across the wavefront).  Both outputs may not alias the inputs.
+ * merged across the wavefront).  In place: residual and normalized may each be
+ * the buffer of value or of update, from its first row on, where the dtypes are
+ * the same; no other overlap, and the two outputs are apart.
  *
  * Replaces the reference's
  *   _residual_layer_norm_kernel        (solution/kernels/norm/triton_residual.py:39-71)        fp32 stream
@@ -378,8 +380,10 @@ int sah_qkv_launch_supported(int block_m, int block_n, int block_k, int num_warp
  *   default path (solution/transformer.py:727-730, 1515-1644)
  * x: [rows, in_features] with row stride x_row_stride; weight: [width,
  * in_features] contiguous; bias, gamma, beta: [width] or NULL (0, 1, 0);
- * value, residual, normalized: [rows, width] contiguous, residual and
- * normalized not aliasing any input.  Shared dtype SAH_DTYPE_BF16 or
+ * value, residual, normalized: [rows, width] contiguous.  In place: residual
+ * and normalized may each be the buffer of value, or of an x of in_features and
+ * x_row_stride == width, from its first row on; no other overlap, and the two
+ * outputs are apart.  Shared dtype SAH_DTYPE_BF16 or
  * SAH_DTYPE_F16; norm_kind SAH_NORM_LAYER or SAH_NORM_RMS.  width 512 or
  * 1024, in_features a multiple of 64, x_row_stride a multiple of 8; tensors
  * 16-byte aligned, bias 8-byte.  Launch: block_rows = 65536 / width, num_warps = 8

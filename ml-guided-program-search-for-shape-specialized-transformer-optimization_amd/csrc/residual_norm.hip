@@ -50,12 +50,16 @@ struct VecIO {
 // ONE_ROW: rows_per_wave == 1, compiled as straight-line code, so the affine
 // parameters stay packed until they are used (55 instead of 77 VGPRs at width
 // 1024 bf16: 8 instead of 6 waves per SIMD, 26.6 -> 25.6 us for 16384 rows).
+// In place: an output may be value or update of its own dtype, row for row
+// (sah_linear_residual_norm passes the update in an output).  A wave loads
+// its row whole before it stores any of it, and every lane stores the columns
+// it loaded; so these four pointers are not __restrict__, and the order of
+// loads and stores below is part of the contract.
 template <typename TX, typename TU, typename TY, typename TP, int ITERS, bool HAS_RES, bool ONE_ROW,
           int VEC = 16 / sizeof(TX)>
 __global__ __launch_bounds__(512) void norm_kernel(
-    const TX* __restrict__ value, const TU* __restrict__ update,
-    const TP* __restrict__ weight, const TP* __restrict__ bias,
-    TX* __restrict__ residual, TY* __restrict__ normalized, int64_t rows,
+    const TX* value, const TU* update, const TP* __restrict__ weight,
+    const TP* __restrict__ bias, TX* residual, TY* normalized, int64_t rows,
     float eps, int rows_per_wave, int rms) {
   constexpr int WIDTH = ITERS * kWave * VEC;
   constexpr int N = ITERS * VEC;

@@ -227,3 +227,37 @@ def test_outputs_over_inputs_through_the_c_abi(gpu_device, residual_on, normaliz
     _library.check_status(status, "sah_linear_residual_norm")
     torch.cuda.synchronize()
     assert torch.equal(residual, r_ref) and torch.equal(normalized, y_ref)
+
+
+@pytest.mark.parametrize("residual_on,normalized_on", [("x", None), (None, "x"), ("x", "value")])
+@pytest.mark.parametrize("norm_kind", ["layer", "rms"])
+def test_outputs_over_x_through_the_c_abi(gpu_device, residual_on, normalized_on, norm_kind):
+    """The other in-place forms (outputs over x), fp16 at width 1024, ragged
+    rows, both norms: the separate buffers' results bit for bit."""
+
+    from solution.kernels.boundary import block_rows_for
+    from solution.kernels.hip import _library
+
+    width, rows, dtype = 1024, 201, torch.float16
+    kind = _library.SAH_NORM_LAYER if norm_kind == "layer" else _library.SAH_NORM_RMS
+    g = torch.Generator().manual_seed(13)
+    x = torch.randint(-2, 3, (rows, width), generator=g).to(dtype).to(gpu_device)
+    w = (torch.randint(-2, 3, (width, width), generator=g).float() / 16).to(dtype).to(gpu_device)
+    value = torch.randn(rows, width, generator=g).to(dtype).to(gpu_device)
+
+    def call(source, stream, r, y):
+        status = _library.load_library().sah_linear_residual_norm(
+            source.data_ptr(), w.data_ptr(), None, stream.data_ptr(), None, None, r.data_ptr(), y.data_ptr(), rows,
+            width, width, width, 1e-5, _library.dtype_code(dtype), kind, block_rows_for(width), 8,
+            _library.stream_handle(gpu_device),
+        )
+        _library.check_status(status, "sah_linear_residual_norm")
+
+    expected = torch.empty_like(value), torch.empty_like(value)
+    call(x, value, *expected)
+    buffers = {"x": x.clone(), "value": value.clone()}
+    r = buffers[residual_on] if residual_on else torch.empty_like(value)
+    y = buffers[normalized_on] if normalized_on else torch.empty_like(value)
+    call(buffers["x"], buffers["value"], r, y)
+    torch.cuda.synchronize()
+    assert torch.equal(r, expected[0]) and torch.equal(y, expected[1])

@@ -226,3 +226,46 @@ def test_ineligible_inputs_raise(gpu_device):
             module.hip_residual_layer_norm(value, value, layer_norm)
         with pytest.raises(ValueError):
             module.hip_residual_layer_norm(value, value, layer_norm, block_rows=3, num_warps=2)
+
+
+@pytest.mark.parametrize("value_dtype,update_dtype", [
+    (torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16), (torch.float32, torch.float32),
+    (torch.float32, torch.float16),
+])
+@pytest.mark.parametrize("width", [128, 256, 1024, 4096])
+@pytest.mark.parametrize("block_rows,num_warps", [(4, 4), (16, 4), (64, 1)])
+def test_in_place_through_the_c_abi(gpu_device, value_dtype, update_dtype, width, block_rows, num_warps):
+    """Each output over value or update (one row and several rows per wave, a
+    partial last block) gives the separate buffers' results bit for bit."""
+
+    from solution.kernels.hip import _library
+
+    rows = 83
+    normalized_dtype = update_dtype
+    g = torch.Generator().manual_seed(width + rows)
+    value = torch.randn(rows, width, generator=g).to(value_dtype).to(gpu_device)
+    update = torch.randn(rows, width, generator=g).to(update_dtype).to(gpu_device)
+    ln = _layer_norm(width, value_dtype, 5, gpu_device)
+    code = _library.dtype_code
+
+    def call(v, u, r, y):
+        status = _library.load_library().sah_residual_norm(
+            v.data_ptr(), u.data_ptr(), ln.weight.data_ptr(), ln.bias.data_ptr(), r.data_ptr(), y.data_ptr(), rows,
+            width, 1e-5, code(value_dtype), code(update_dtype), code(normalized_dtype), code(value_dtype),
+            _library.SAH_NORM_LAYER, block_rows, num_warps, _library.stream_handle(gpu_device),
+        )
+        _library.check_status(status, "sah_residual_norm")
+
+    expected = torch.empty_like(value), torch.empty(rows, width, dtype=normalized_dtype, device=gpu_device)
+    call(value, update, *expected)
+    same = value_dtype == update_dtype
+    for residual_on, normalized_on in [("value", None), (None, "update"), ("value", "update")] + (
+        [("update", None), (None, "value"), ("update", "value")] if same else []
+    ):
+        v, u = value.clone(), update.clone()
+        buffers = {"value": v, "update": u}
+        r = buffers[residual_on] if residual_on else torch.empty_like(expected[0])
+        y = buffers[normalized_on] if normalized_on else torch.empty_like(expected[1])
+        call(v, u, r, y)
+        torch.cuda.synchronize()
+        assert torch.equal(r, expected[0]) and torch.equal(y, expected[1]), (residual_on, normalized_on)
