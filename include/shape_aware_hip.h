@@ -369,7 +369,8 @@ int sah_qkv_launch_supported(int block_m, int block_n, int block_k, int num_warp
  *   residual   = round_to(dtype, value + update)
  *   normalized = round_to(dtype, norm(residual) * gamma + beta)
  * Two launches on the stream (the projection leaves the rounded update in an
- * output buffer, the norm reads it back in place); no workspace.  The residual
+ * output buffer, the norm reads it back in place), or one kernel where a short
+ * in_features and the row count make it faster; no workspace.  The residual
  * and norm arithmetic are those of sah_residual_norm (statistics in fp32 over
  * the rounded residual).
  *

@@ -12,7 +12,7 @@
 // path does (the projection's output, then sah_residual_norm); the residual
 // and norm arithmetic are those of csrc/residual_norm.hip.
 //
-// MI355X formulation: two launches on the caller's stream.  The projection
+// MI355X formulation, in general: two launches on the caller's stream.  The projection
 // runs on the tile kernels (linear_tiles.hip) and leaves the rounded update in
 // one of the two output buffers; the fused norm kernel (residual_norm.hip)
 // then reads it back in place: a wavefront reads its whole row before it
@@ -25,8 +25,9 @@
 //   20000 x 4096 -> 1024   558 ->  205 us     804 x 1024 -> 1024   71 -> 19 us
 //   200000 x 1024 -> 1024 1155 ->  672 us  200000 x 4096 -> 1024 3700 -> 1620 us
 //
-// The one-kernel form remains for outputs that both overlap an input, where
-// neither can hold the update.  In it:
+// The one-kernel form serves a short K whose row blocks fill one or two rounds
+// of the CUs (one_kernel_pays), and outputs that both are inputs' buffers,
+// where neither can hold the update.  In it:
 //  * One workgroup (8 wavefronts) owns BM = 65536 / D whole rows, so the row
 //    statistics never leave the workgroup.  Wave w computes output columns
 //    [w D/8, (w+1) D/8) of all BM rows: 8 accumulator blocks of 32 x 32
@@ -286,6 +287,32 @@ bool overlap(const void* a, int64_t a_bytes, const void* b, int64_t b_bytes) {
   return a != nullptr && b != nullptr && pa < pb + (uintptr_t)b_bytes && pb < pa + (uintptr_t)a_bytes;
 }
 
+// Whether the one-kernel form is the faster one.  Its time is rounds of the 256
+// CUs, BM rows each, about alike for one row and for BM; the two launches pay
+// per row.  So it is for a short K, where W is soon streamed, and row counts that
+// nearly fill their rounds.  Estimates in us, fitted to both forms over K 64-2048
+// and 4096-200000 rows (the form taken is at most 5% behind the better one);
+// measured (bf16, us, one kernel / two launches):
+//   32768 x 64 -> 512   24.1 / 35.1    16384 x 64 -> 1024   25.2 / 37.1
+//   65536 x 64 -> 512   44.6 / 62.9    32768 x 64 -> 1024   46.3 / 62.1
+//   32768 x 512 -> 512  38.9 / 44.9    16384 x 256 -> 1024  36.7 / 40.0
+//   20000 x 512 -> 512  35.9 / 34.9    10000 x 256 -> 1024  about even
+//   65536 x 512 -> 512  85.8 / 85.5    32768 x 1024 -> 512  56.6 / 55.6
+// and for a handful of rows and one K step, 1 x 64 -> 512, 6.2 / 7.0.
+bool one_kernel_pays(int64_t rows, int64_t k, int64_t width) {
+  const int64_t steps = k / kLnBK;
+  const bool wide = width == 1024;
+  if (!wide && steps == 1 && rows <= 8) return true;
+  if (steps > (wide ? 4 : 8)) return false;
+  const int64_t rounds = ceil_div(rows, 65536 / width * 256);
+  const int64_t most = steps <= (wide ? 1 : 2) ? 3 : steps <= 6 ? 2 : 1;
+  if (rounds > most) return false;
+  const double s = (double)steps, thousands = 1e-3 * (double)rows;
+  const double one = (double)rounds * (wide ? 19.0 + 3.5 * s : 18.0 + 2.4 * s);
+  const double two = wide ? 11.0 + thousands * (1.7 + 0.06 * s) : 10.0 + thousands * (0.9 + 0.04 * s);
+  return one < two;
+}
+
 template <typename T, int D>
 int launch_linear_norm(const LinearNormParams& prm, hipStream_t stream) {
   const int64_t blocks = (prm.rows + LnShape<D>::BM - 1) / LnShape<D>::BM;
@@ -349,7 +376,8 @@ extern "C" int sah_linear_residual_norm(const void* x, const void* weight, const
     return fail(SAH_ERR_INVALID_ARGUMENT,
                 "sah_linear_residual_norm: tensors must be 16-byte aligned (bias 8-byte)");
   // Two launches where an output can hold the update: one that overlaps no
-  // input (the reader of the next launch is the other output's too).
+  // input (the reader of the next launch is the other output's too).  With both
+  // outputs clear of the inputs the faster form is free to be taken.
   const int64_t row_bytes = width * 2, out_bytes = rows * row_bytes;
   const int64_t x_bytes = ((rows - 1) * x_row_stride + in_features) * 2;
   auto holds_update = [&](const void* out) {
@@ -357,8 +385,9 @@ extern "C" int sah_linear_residual_norm(const void* x, const void* weight, const
            !overlap(out, out_bytes, weight, in_features * row_bytes) && !overlap(out, out_bytes, bias, row_bytes) &&
            !overlap(out, out_bytes, gamma, row_bytes) && !overlap(out, out_bytes, beta, row_bytes);
   };
-  void* update = holds_update(normalized) ? normalized : holds_update(residual) ? residual : nullptr;
-  if (update != nullptr) {
+  const bool clear_n = holds_update(normalized), clear_r = holds_update(residual);
+  void* update = clear_n ? normalized : clear_r ? residual : nullptr;
+  if (update != nullptr && !(clear_n && clear_r && one_kernel_pays(rows, in_features, width))) {
     const int status = sah_linear(x, weight, bias, update, rows, in_features, width, x_row_stride, width, dtype,
                                   SAH_ACTIVATION_NONE, 256, 256, 64, 8, 2, stream);
     if (status != SAH_OK) return status;

@@ -261,3 +261,36 @@ def test_outputs_over_x_through_the_c_abi(gpu_device, residual_on, normalized_on
     call(buffers["x"], buffers["value"], r, y)
     torch.cuda.synchronize()
     assert torch.equal(r, expected[0]) and torch.equal(y, expected[1])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,in_features,width", [
+    # the one-kernel form: a few rows and one K step; one, two and three rounds of the
+    # CUs, ragged; the two-launch form on the other side of each line
+    (1, 64, 512), (8, 64, 512), (9, 64, 512), (32767, 64, 512), (61000, 128, 512), (32700, 512, 512), (33000, 512, 512),
+    (30001, 576, 512), (16300, 256, 1024), (16300, 320, 1024), (32001, 128, 1024), (16385, 64, 1024), (40000, 64, 1024),
+])
+def test_both_forms_at_the_lines_of_their_rule(gpu_device, rows, in_features, width, dtype):
+    """Integer operands make the update exact in fp32 whatever the order of its
+    sum, so residual and normalized equal the unfused boundary's bit for bit in
+    either form."""
+
+    from solution.kernels.boundary import block_rows_for, hip_linear_residual_norm
+    from solution.kernels.norm.hip_residual import hip_residual_layer_norm
+
+    print(f"boundary {rows}x{in_features}->{width} {dtype}", flush=True)
+    g = torch.Generator(device=gpu_device).manual_seed(rows + in_features)
+    def integers(low, high, *shape):
+        return torch.randint(low, high, shape, generator=g, device=gpu_device).float()
+
+    x = integers(-2, 3, 1, rows, in_features).to(dtype)
+    w = (integers(-2, 3, width, in_features) / 16).to(dtype)
+    b = (integers(-64, 65, width) / 8).to(dtype)
+    value = torch.randn(1, rows, width, generator=g, device=gpu_device).to(dtype)
+    update = F.linear(x.double(), w.double(), b.double()).to(dtype)
+    ln = _layer_norm(width, dtype, gpu_device, seed=rows)
+    with torch.inference_mode():
+        r, y, _ = hip_linear_residual_norm(x, w, b, value, ln, block_rows=block_rows_for(width), num_warps=8)
+        r_ref, y_ref, _ = hip_residual_layer_norm(value, update, ln)
+    torch.cuda.synchronize()
+    assert torch.equal(r, r_ref) and torch.equal(y, y_ref)
