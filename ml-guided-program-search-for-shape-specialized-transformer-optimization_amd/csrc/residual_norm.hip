@@ -181,11 +181,20 @@ struct NormArgs {
   hipStream_t stream;
 };
 
+// A grid holds fewer than 2^32 work items (the launch drops the rest without an
+// error): so many rows take more rows per wave, with the same results.
+int launched_block_rows(const NormArgs& a) {
+  int block_rows = a.block_rows;
+  while (ceil_div(a.rows, block_rows) * (a.num_warps * kWave) > (int64_t)UINT32_MAX) block_rows *= 2;
+  return block_rows;
+}
+
 template <typename TX, typename TU, typename TY, typename TP, bool HAS_RES, int NARROW>
 int launch_narrow(const NormArgs& a) {
-  const int rows_per_wave = a.block_rows / a.num_warps;
-  const int64_t grid = ceil_div(a.rows, a.block_rows);
-  if (grid > INT32_MAX) return fail(SAH_ERR_UNSUPPORTED, "too many rows");
+  if (ceil_div(a.rows, a.block_rows) > INT32_MAX) return fail(SAH_ERR_UNSUPPORTED, "too many rows");
+  const int block_rows = launched_block_rows(a);
+  const int rows_per_wave = block_rows / a.num_warps;
+  const int64_t grid = ceil_div(a.rows, block_rows);
   const dim3 block(a.num_warps * kWave);
   if (rows_per_wave == 1)
     hipLaunchKernelGGL((norm_kernel<TX, TU, TY, TP, 1, HAS_RES, true, NARROW>), dim3(grid), block, 0,
@@ -214,9 +223,10 @@ int launch_typed(const NormArgs& a) {
                 (long long)a.width, VEC == 8 ? "256 " : "", (long long)per_iter);
   }
   const int64_t iters = a.width / per_iter;
-  const int rows_per_wave = a.block_rows / a.num_warps;
-  const int64_t grid = ceil_div(a.rows, a.block_rows);
-  if (grid > INT32_MAX) return fail(SAH_ERR_UNSUPPORTED, "too many rows");
+  if (ceil_div(a.rows, a.block_rows) > INT32_MAX) return fail(SAH_ERR_UNSUPPORTED, "too many rows");
+  const int block_rows = launched_block_rows(a);
+  const int rows_per_wave = block_rows / a.num_warps;
+  const int64_t grid = ceil_div(a.rows, block_rows);
   const dim3 block(a.num_warps * kWave);
   const TX* value = static_cast<const TX*>(a.value);
   const TU* update = static_cast<const TU*>(a.update);

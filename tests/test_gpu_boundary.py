@@ -294,3 +294,48 @@ def test_both_forms_at_the_lines_of_their_rule(gpu_device, rows, in_features, wi
         r_ref, y_ref, _ = hip_residual_layer_norm(value, update, ln)
     torch.cuda.synchronize()
     assert torch.equal(r, r_ref) and torch.equal(y, y_ref)
+
+
+def test_more_rows_than_a_wave_each_can_launch(gpu_device):
+    """2^26 + 5 rows of width 512: with one wave per row the norm's launch would
+    be 2^32 work items, which a grid does not hold.  In place (residual over
+    value), 136 GiB; sampled rows equal the same rows of a small call bit for
+    bit (the projection's tiles all sum K in one order)."""
+
+    from solution.kernels.boundary import block_rows_for
+    from solution.kernels.hip import _library
+
+    rows, width, in_features, dtype = (1 << 26) + 5, 512, 64, torch.bfloat16
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info(gpu_device)[0] < 150 << 30:
+        pytest.skip("needs 150 GiB of free GPU memory")
+    print(f"boundary {rows}x{in_features}->{width}", flush=True)
+    g = torch.Generator().manual_seed(1)
+    w = (torch.randn(width, in_features, generator=g) / 8).to(dtype).to(gpu_device)
+    b = torch.randn(width, generator=g).to(dtype).to(gpu_device)
+    ln = _layer_norm(width, dtype, gpu_device, seed=2)
+    pick = torch.cat([torch.arange(n, n + 64) for n in (0, 1 << 25, (1 << 26) - 66, rows - 64)]).unique().to(gpu_device)
+    xs = torch.randn(len(pick), in_features, generator=g).to(dtype).to(gpu_device)
+    vs = torch.randn(len(pick), width, generator=g).to(dtype).to(gpu_device)
+
+    def call(x, value, residual, normalized, n):
+        status = _library.load_library().sah_linear_residual_norm(
+            x.data_ptr(), w.data_ptr(), b.data_ptr(), value.data_ptr(), ln.weight.data_ptr(), ln.bias.data_ptr(),
+            residual.data_ptr(), normalized.data_ptr(), n, in_features, width, in_features, ln.eps,
+            _library.dtype_code(dtype), _library.SAH_NORM_LAYER, block_rows_for(width), 8,
+            _library.stream_handle(gpu_device),
+        )
+        _library.check_status(status, "sah_linear_residual_norm")
+
+    expected = torch.empty_like(vs), torch.empty_like(vs)
+    call(xs, vs, *expected, len(pick))
+    x = torch.zeros(rows, in_features, dtype=dtype, device=gpu_device)
+    value = torch.zeros(rows, width, dtype=dtype, device=gpu_device)
+    normalized = torch.empty(rows, width, dtype=dtype, device=gpu_device)
+    x[pick], value[pick] = xs, vs
+    call(x, value, value, normalized, rows)
+    torch.cuda.synchronize()
+    same = torch.equal(value[pick], expected[0]) and torch.equal(normalized[pick], expected[1])
+    del x, value, normalized
+    torch.cuda.empty_cache()
+    assert same
