@@ -43,11 +43,18 @@ __global__ __launch_bounds__(512) void gelu_kernel(const T* x, T* y, int64_t n) 
 
 template <typename T, int CPT>
 int launch_gelu(const void* x, void* y, int64_t n, int threads, hipStream_t stream) {
+  // A grid holds fewer than 2^32 work items (the launch drops the rest without an
+  // error): more elements go out as several launches.
   const int64_t per_block = (int64_t)threads * CPT * 8;
-  const int64_t blocks = (n + per_block - 1) / per_block;
-  hipLaunchKernelGGL((gelu_kernel<T, CPT>), dim3((unsigned)blocks), dim3(threads), 0, stream,
-                     static_cast<const T*>(x), static_cast<T*>(y), n);
-  return check_hip(hipGetLastError(), "gelu kernel launch");
+  const int64_t per_launch = (int64_t)UINT32_MAX / threads * per_block;
+  for (int64_t first = 0; first < n; first += per_launch) {
+    const int64_t count = n - first < per_launch ? n - first : per_launch;
+    hipLaunchKernelGGL((gelu_kernel<T, CPT>), dim3((unsigned)ceil_div(count, per_block)), dim3(threads), 0, stream,
+                       static_cast<const T*>(x) + first, static_cast<T*>(y) + first, count);
+    const int status = check_hip(hipGetLastError(), "gelu kernel launch");
+    if (status != SAH_OK) return status;
+  }
+  return SAH_OK;
 }
 
 template <typename T>

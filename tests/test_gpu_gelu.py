@@ -118,3 +118,31 @@ def test_ineligible_and_bad_launch_raise(gpu_device):
         prevalidated_hip_exact_gelu(x, block_size=256)
     with pytest.raises(RuntimeError, match="output buffer"):
         prevalidated_hip_exact_gelu(x, out=torch.zeros(8, device=gpu_device, dtype=torch.bfloat16))
+
+
+def test_more_elements_than_one_launch_holds(gpu_device):
+    """2^35 + 2^20 + 5 elements in place (64 GiB) with 8 elements a thread, the
+    model's launch: one grid holds fewer than 2^32 threads.  Samples from the
+    start, about the line and the end equal a small call's."""
+
+    from solution.kernels.ffn import prevalidated_hip_exact_gelu
+
+    n = (1 << 35) + (1 << 20) + 5
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info(gpu_device)[0] < 80 << 30:
+        pytest.skip("needs 80 GiB of free GPU memory")
+    print(f"gelu {n}", flush=True)
+    g = torch.Generator().manual_seed(4)
+    sample = torch.randn(4096, generator=g).to(torch.bfloat16).to(gpu_device)
+    value = torch.zeros(n, dtype=torch.bfloat16, device=gpu_device)
+    starts = (0, (1 << 35) - 4096 - 2048, 1 << 35, n - 4096)
+    for first in starts:
+        value[first : first + 4096] = sample
+    with torch.inference_mode():
+        expected, _ = prevalidated_hip_exact_gelu(sample)
+        out, _ = prevalidated_hip_exact_gelu(value, num_warps=8, out=value)
+    torch.cuda.synchronize()
+    same = [torch.equal(out[first : first + 4096], expected) for first in starts]
+    del value, out
+    torch.cuda.empty_cache()
+    assert all(same), same
