@@ -11,6 +11,7 @@ from __future__ import annotations
 
 import torch
 from torch import nn
+from torch.autograd import forward_ad
 
 from ..hip._library import (
     SAH_ACTIVATION_GELU_EXACT,
@@ -62,6 +63,8 @@ def _is_plain(module: nn.Linear, value: torch.Tensor) -> bool:
     if torch.compiler.is_compiling() or torch.jit.is_tracing():
         return False
     if torch.is_grad_enabled() or torch.is_autocast_enabled("cuda"):
+        return False
+    if forward_ad._current_level >= 0:  # dual tensors carry tangents under no_grad too
         return False
     if type(value) is not torch.Tensor or type(module.weight) not in (nn.Parameter, torch.Tensor):
         return False

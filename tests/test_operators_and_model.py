@@ -162,3 +162,20 @@ def test_model_projection_rule():
     linear = torch.nn.Linear(256, 256)
     with torch.no_grad():
         assert project(linear, torch.zeros(2, 8, 256)) is None
+
+
+def test_model_projection_leaves_observed_calls_to_the_module():
+    """A call of more than one F.linear on plain tensors is not plain."""
+
+    from solution.kernels.projection.hip_linear import _is_plain
+
+    linear = torch.nn.Linear(128, 32)
+    value = torch.randn(4, 128)
+    with torch.no_grad():
+        assert _is_plain(linear, value)
+        # forward-mode tangents pass through F.linear under no_grad
+        with torch.autograd.forward_ad.dual_level():
+            dual = torch.autograd.forward_ad.make_dual(value, torch.ones_like(value))
+            assert torch.autograd.forward_ad.unpack_dual(linear(dual)).tangent is not None
+            assert not _is_plain(linear, dual)
+        assert _is_plain(linear, value)
