@@ -72,6 +72,8 @@ def _is_plain(module: nn.Linear, value: torch.Tensor) -> bool:
         return False
     if module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__:
         return False
+    if type(module).forward is not nn.Linear.forward or type(module).__call__ is not nn.Module.__call__:
+        return False
     registry = nn.modules.module
     if registry._global_forward_hooks or registry._global_forward_pre_hooks:
         return False

@@ -179,3 +179,13 @@ def test_model_projection_leaves_observed_calls_to_the_module():
             assert torch.autograd.forward_ad.unpack_dual(linear(dual)).tangent is not None
             assert not _is_plain(linear, dual)
         assert _is_plain(linear, value)
+        # subclasses that put something before or after the product
+        class Scaled(torch.nn.Linear):
+            def forward(self, value):
+                return 2 * super().forward(value)
+
+        class Called(torch.nn.Linear):
+            def __call__(self, value):
+                return 2 * super().__call__(value)
+
+        assert not _is_plain(Scaled(128, 32), value) and not _is_plain(Called(128, 32), value)
