@@ -66,10 +66,11 @@ def _is_plain(module: nn.Linear, value: torch.Tensor) -> bool:
         return False
     if forward_ad._current_level >= 0:  # dual tensors carry tangents under no_grad too
         return False
-    if type(value) is not torch.Tensor or type(module.weight) not in (nn.Parameter, torch.Tensor):
+    if type(value) is not torch.Tensor:
         return False
-    if module.bias is not None and type(module.bias) not in (nn.Parameter, torch.Tensor):
-        return False
+    for parameter in (module._parameters["weight"], module._parameters["bias"]):
+        if parameter is not None and type(parameter) not in (nn.Parameter, torch.Tensor):
+            return False
     if module._forward_hooks or module._forward_pre_hooks or "forward" in module.__dict__:
         return False
     if type(module).forward is not nn.Linear.forward or type(module).__call__ is not nn.Module.__call__:
@@ -89,7 +90,11 @@ def project(module: nn.Linear, value: torch.Tensor, *, gelu: bool = False) -> to
     kernel, or None where it does not serve the call (size, type, layout, or a
     call that something observes)."""
 
-    weight, bias = module.weight, module.bias
+    # as registered: reading a parametrized weight computes it (spectral_norm
+    # takes a power iteration each time), which is for the module to do once
+    weight, bias = module._parameters.get("weight"), module._parameters.get("bias")
+    if weight is None or "bias" not in module._parameters:
+        return None
     dtype = value.dtype
     out_features, in_features = weight.shape
     if not value.is_cuda or value.ndim < 2 or value.shape[-1] != in_features:

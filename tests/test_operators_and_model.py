@@ -189,3 +189,24 @@ def test_model_projection_leaves_observed_calls_to_the_module():
                 return 2 * super().__call__(value)
 
         assert not _is_plain(Scaled(128, 32), value) and not _is_plain(Called(128, 32), value)
+
+
+def test_model_projection_does_not_evaluate_a_parametrized_weight():
+    from solution.kernels.projection.hip_linear import project
+
+    class Counted(torch.nn.Module):
+        calls = 0
+
+        def forward(self, weight):
+            Counted.calls += 1
+            return weight
+
+    linear = torch.nn.Linear(128, 32)
+    for name in ("weight", "bias"):
+        torch.nn.utils.parametrize.register_parametrization(linear, name, Counted())
+    Counted.calls = 0
+    with torch.no_grad():
+        assert project(linear, torch.zeros(4, 128)) is None
+        assert Counted.calls == 0
+        linear(torch.zeros(4, 128))
+    assert Counted.calls == 2
