@@ -265,22 +265,10 @@ class _FP16ShadowLinear(nn.Linear):
         self._fp16_shadow_weight = None
         self._fp16_shadow_bias = None
 
-    def forward_backend(
-        self, value: torch.Tensor, backend: ProjectionBackend, *, hip: bool = False
-    ) -> torch.Tensor:
-        """The projection by ``backend``.  ``hip`` (the programs on the HIP
-        attention): a small fp32 projection may run on the gfx950 kernel, at
-        the sizes where it beats the library GEMM."""
-
+    def forward_backend(self, value: torch.Tensor, backend: ProjectionBackend) -> torch.Tensor:
         if backend is ProjectionBackend.INPUT_DTYPE:
             if value.dtype != self.weight.dtype:
                 value = value.to(self.weight.dtype)
-            if hip:
-                from .kernels.projection.hip_linear import project
-
-                output = project(self, value)
-                if output is not None:
-                    return output
             return self(value)
         if backend is ProjectionBackend.AUTOCAST_FP16:
             with torch.autocast(device_type=value.device.type, dtype=torch.float16, enabled=True):
@@ -291,6 +279,32 @@ class _FP16ShadowLinear(nn.Linear):
                 raise RuntimeError("FP16 shadow weights must be materialized before use")
             return F.linear(value.to(torch.float16), weight, self._fp16_shadow_bias)
         raise AssertionError(f"unhandled projection backend: {backend}")
+
+
+def _hip_projection(
+    linear: nn.Module, value: torch.Tensor, backend: ProjectionBackend, plan: ExecutionPlan, *, gelu: bool = False
+) -> torch.Tensor | None:
+    """A small fp32 projection, with ``gelu`` the exact GELU of it, on the gfx950
+    kernel: in the programs on the HIP attention, at the sizes where it beats
+    the library GEMM, and only in place of this file's own projection (a module
+    put there by the user runs as it is).  None otherwise."""
+
+    if not plan.uses_hip_attention or backend is not ProjectionBackend.INPUT_DTYPE:
+        return None
+    if type(linear) is not _FP16ShadowLinear or "forward_backend" in linear.__dict__:
+        return None
+    from .kernels.projection.hip_linear import project
+
+    if value.dtype != linear.weight.dtype:
+        value = value.to(linear.weight.dtype)
+    return project(linear, value, gelu=gelu)
+
+
+def _project(
+    linear: nn.Module, value: torch.Tensor, backend: ProjectionBackend, plan: ExecutionPlan
+) -> torch.Tensor:
+    output = _hip_projection(linear, value, backend, plan)
+    return linear.forward_backend(value, backend) if output is None else output
 
 
 class _SelfAttention(nn.Module):
@@ -371,7 +385,7 @@ class _SelfAttention(nn.Module):
                 observation.qkv_materializations.append(plan.qkv_materialization.value)
                 observation.qkv_launches.append(_launch_dict(plan.qkv_launch))
         else:
-            packed = self.qkv_proj.forward_backend(value, plan.qkv_projection_backend, hip=plan.uses_hip_attention)
+            packed = _project(self.qkv_proj, value, plan.qkv_projection_backend, plan)
             qkv_dtype = packed.dtype
             query, key, projected = split_qkv(
                 packed,
@@ -434,9 +448,7 @@ class _SelfAttention(nn.Module):
                 f"attention bridge {plan.attention_output_bridge.value} is not executable here"
             )
         output = (
-            self.out_proj.forward_backend(
-                context, plan.attention_output_projection_backend, hip=plan.uses_hip_attention
-            )
+            _project(self.out_proj, context, plan.attention_output_projection_backend, plan)
             if project
             else context
         )
@@ -541,9 +553,7 @@ class _TransformerBlock(nn.Module):
             launch = plan.ffn_launch
             if launch is None:
                 raise RuntimeError("HIP Exact-GELU plan is missing launch parameters")
-            projected = self.ffn_in.forward_backend(
-                normalized, plan.ffn_input_projection_backend, hip=plan.uses_hip_attention
-            )
+            projected = self.ffn_in.forward_backend(normalized, plan.ffn_input_projection_backend)
             input_compute_dtype = _dtype_name(projected.dtype)
             # in place: the projection is a temporary of this block
             hidden, marker = prevalidated_hip_exact_gelu(
@@ -553,12 +563,10 @@ class _TransformerBlock(nn.Module):
                 marker, expected_marker=HIP_EXACT_GELU_BACKEND, planned_backend=plan.ffn_backend.value
             )
         else:
-            hidden = None
-            if plan.uses_hip_attention and plan.ffn_input_projection_backend is ProjectionBackend.INPUT_DTYPE:
-                from .kernels.projection.hip_linear import project as hip_project
-
-                # a small fp32 projection and its GELU as one launch
-                hidden = hip_project(self.ffn_in, normalized, gelu=True)
+            # a small fp32 projection and its GELU as one launch
+            hidden = _hip_projection(
+                self.ffn_in, normalized, plan.ffn_input_projection_backend, plan, gelu=True
+            )
             if hidden is not None:
                 input_compute_dtype = _dtype_name(hidden.dtype)
             else:
@@ -568,9 +576,7 @@ class _TransformerBlock(nn.Module):
                     projected = projected.float()
                 hidden = F.gelu(projected, approximate="none")
         update = (
-            self.ffn_out.forward_backend(
-                hidden, plan.ffn_output_projection_backend, hip=plan.uses_hip_attention
-            )
+            _project(self.ffn_out, hidden, plan.ffn_output_projection_backend, plan)
             if project
             else hidden
         )

@@ -461,3 +461,34 @@ def test_default_resolution_selects_the_published_registry_entry(gpu_device):
     with torch.inference_mode():
         model(x)
     assert model.describe_execution_path()["planned_config_id"] == published.config_id
+
+
+@pytest.mark.parametrize("name", ["attention.qkv_proj", "attention.out_proj", "ffn_in", "ffn_out"])
+def test_replaced_projection_of_an_fp32_model_runs_as_it_is(gpu_device, name):
+    """A projection that overrides forward_backend (its own kernel, an adapter)
+    is called for, with the two arguments of the method, where this file's own
+    projections run on the small fp32 kernel."""
+
+    from solution.config import FFNBackend, hip_config
+
+    config = TransformerConfig(2, 64, 256, 4, 1024, 1, True)
+    state = xavier_init_weights(config, seed=4)
+    model = _model(config, state, gpu_device, torch.float32)
+    model.configure_execution(config=hip_config(ffn=FFNBackend.TORCH))
+    x = generate_input(config, seed=4).to(gpu_device)
+    with torch.inference_mode():
+        expected = model(x)
+        owner = [module for path, module in model.named_modules() if path.endswith(name)]
+        assert len(owner) == 1
+        calls = []
+
+        class Observed(type(owner[0])):
+            def forward_backend(self, value, backend):
+                calls.append(backend)
+                return super().forward_backend(value, backend)
+
+        owner[0].__class__ = Observed
+        output = model(x)
+    torch.cuda.synchronize()
+    assert len(calls) == 1
+    _check(expected.cpu(), output, torch.float32, f"replaced {name}")
