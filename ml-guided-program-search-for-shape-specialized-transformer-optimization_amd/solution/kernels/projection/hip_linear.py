@@ -58,10 +58,8 @@ def _serves(rows: int, in_features: int, out_features: int, dtype: torch.dtype) 
 
 def _is_plain(module: nn.Linear, value: torch.Tensor) -> bool:
     """Whether calling ``module`` is no more than one F.linear on plain
-    tensors: nothing observes, differentiates, casts or traces the call."""
+    tensors: nothing observes, differentiates or casts the call."""
 
-    if torch.compiler.is_compiling() or torch.jit.is_tracing():
-        return False
     if torch.is_grad_enabled() or torch.is_autocast_enabled("cuda"):
         return False
     if forward_ad._current_level >= 0:  # dual tensors carry tangents under no_grad too
@@ -90,6 +88,9 @@ def project(module: nn.Linear, value: torch.Tensor, *, gelu: bool = False) -> to
     kernel, or None where it does not serve the call (size, type, layout, or a
     call that something observes)."""
 
+    # first, so that a trace holds no guard on what follows (the sizes)
+    if torch.compiler.is_compiling() or torch.jit.is_tracing():
+        return None
     # as registered: reading a parametrized weight computes it (spectral_norm
     # takes a power iteration each time), which is for the module to do once
     weight, bias = module._parameters.get("weight"), module._parameters.get("bias")

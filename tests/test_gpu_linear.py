@@ -264,3 +264,27 @@ def test_model_projection_takes_what_it_serves(gpu_device):
         handle.remove()
         assert project(linear, value) is not None
     assert project(linear, value) is None  # grad enabled
+
+
+def test_model_projection_leaves_no_guard_in_a_compiled_caller(gpu_device):
+    """Under torch.compile the call is F.linear whatever the size: a caller of a
+    dynamic row count compiles once, on both sides of the rule's line."""
+
+    from torch._dynamo.testing import CompileCounter
+    from solution.kernels.projection.hip_linear import project
+
+    linear = torch.nn.Linear(256, 256, device=gpu_device)
+    counter = CompileCounter()
+    torch._dynamo.reset()
+
+    @torch.compile(backend=counter, fullgraph=True)
+    def call(value):
+        output = project(linear, value)
+        return linear(value) if output is None else output
+
+    with torch.no_grad():
+        for rows in (64, 250, 5000):
+            value = torch.randn(rows, 256, device=gpu_device)
+            torch._dynamo.mark_dynamic(value, 0)
+            assert torch.equal(call(value), F.linear(value, linear.weight, linear.bias)), rows
+    assert counter.frame_count == 1
