@@ -281,6 +281,10 @@ class _FP16ShadowLinear(nn.Linear):
         raise AssertionError(f"unhandled projection backend: {backend}")
 
 
+def _is_own_projection(linear: nn.Module) -> bool:
+    return type(linear) is _FP16ShadowLinear and "forward_backend" not in linear.__dict__
+
+
 def _hip_projection(
     linear: nn.Module, value: torch.Tensor, backend: ProjectionBackend, plan: ExecutionPlan, *, gelu: bool = False
 ) -> torch.Tensor | None:
@@ -291,18 +295,19 @@ def _hip_projection(
 
     if not plan.uses_hip_attention or backend is not ProjectionBackend.INPUT_DTYPE:
         return None
-    if type(linear) is not _FP16ShadowLinear or "forward_backend" in linear.__dict__:
+    if not _is_own_projection(linear):
         return None
     from .kernels.projection.hip_linear import project
 
-    if value.dtype != linear.weight.dtype:
-        value = value.to(linear.weight.dtype)
     return project(linear, value, gelu=gelu)
 
 
 def _project(
     linear: nn.Module, value: torch.Tensor, backend: ProjectionBackend, plan: ExecutionPlan
 ) -> torch.Tensor:
+    if backend is ProjectionBackend.INPUT_DTYPE and _is_own_projection(linear):
+        if value.dtype != linear.weight.dtype:  # once, for either path
+            value = value.to(linear.weight.dtype)
     output = _hip_projection(linear, value, backend, plan)
     return linear.forward_backend(value, backend) if output is None else output
 

@@ -210,3 +210,26 @@ def test_model_projection_does_not_evaluate_a_parametrized_weight():
         assert Counted.calls == 0
         linear(torch.zeros(4, 128))
     assert Counted.calls == 2
+
+
+@pytest.mark.parametrize("hip", [False, True])
+def test_projection_converts_its_input_once(hip):
+    from types import SimpleNamespace
+
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from solution.config import ProjectionBackend
+    from solution.transformer import _FP16ShadowLinear, _project
+
+    class Conversions(TorchDispatchMode):
+        count = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.count += func is torch.ops.aten._to_copy.default
+            return func(*args, **(kwargs or {}))
+
+    linear = _FP16ShadowLinear(256, 64)
+    plan = SimpleNamespace(uses_hip_attention=hip)
+    with torch.no_grad(), Conversions() as mode:
+        output = _project(linear, torch.ones(4, 256, dtype=torch.float16), ProjectionBackend.INPUT_DTYPE, plan)
+    assert output.dtype == torch.float32 and mode.count == 1
