@@ -225,7 +225,9 @@ typedef enum {
  *     (solution/transformer.py:828-842)
  * x: [rows, in_features] with row stride x_row_stride; weight: [out_features,
  * in_features] contiguous (nn.Linear layout); bias: [out_features]; y: [rows,
- * out_features] with row stride y_row_stride.  x, weight, bias and y share
+ * out_features] with row stride y_row_stride, overlapping no input, but that
+ * with 256 output columns y may be x in place (the same first row and row
+ * stride).  x, weight, bias and y share
  * dtype (SAH_DTYPE_BF16 or SAH_DTYPE_F16).  in_features must be a multiple of
  * 64 and out_features of 256; strides multiples of 8 elements; x, weight and y
  * 16-byte aligned, bias 8-byte aligned.  Launch: (block_m, block_n, block_k,

@@ -9,9 +9,9 @@
 //
 // MI355X formulation: the direct-to-LDS tile kernels of linear_tiles.hip,
 // chosen by size.  The kernel in this file stages its operands through
-// registers and remains for the two cases the others do not take: a LayerNorm
-// applied to x on its way into LDS, and x rows further apart than the
-// direct loads' 32-bit offsets reach.  It is
+// registers and remains for the cases the others do not take: a LayerNorm
+// applied to x on its way into LDS, x rows further apart than the
+// direct loads' 32-bit offsets reach, and y written over x.  It is
 //  * a 256 x 256 output tile per workgroup of 8 wavefronts (2 x 4), each wave
 //    owning 128 rows x 64 columns; K advances 64 at a time through a
 //    double-buffered LDS stage (rows padded by 16 bytes, conflict-free 16-byte
@@ -283,10 +283,25 @@ __global__ __launch_bounds__(kThreads) void linear_kernel(LinearParams p) {
   store_tile<T, EPI, kBM, kBN, 2, 4>(p, smem, m0, n0, acc);
 }
 
+// Whether y shares bytes with x.  At 256 columns the register-staged kernel's
+// one tile per row block reads its x rows before it writes them; the tile
+// kernels may give a row block to several workgroups, or read its rows again.
+bool y_over_x(const LinearParams& p) {
+  const uintptr_t x = reinterpret_cast<uintptr_t>(p.x), y = reinterpret_cast<uintptr_t>(p.y);
+  const uintptr_t x_end = x + (uintptr_t)((p.rows - 1) * p.x_ld + p.k) * 2;
+  const uintptr_t y_end = y + (uintptr_t)((p.rows - 1) * p.y_ld + p.n) * 2;
+  if (y == 0 || x >= y_end || y >= x_end) return false;
+  if (p.x_ld != p.y_ld) return true;
+  // columns of one buffer's rows: apart where y lies in the rest of x's rows
+  const int64_t pitch = p.x_ld * 2;
+  const int64_t at = ((int64_t)(y - x) % pitch + pitch) % pitch;
+  return at < (int64_t)p.k * 2 || at + (int64_t)p.n * 2 > pitch;
+}
+
 template <typename T, int EPI, bool LN = false>
 int launch_linear(const LinearParams& prm, hipStream_t stream) {
   if constexpr (!LN) {
-    if (prm.x_ld <= kMaxTileStride) {
+    if (prm.x_ld <= kMaxTileStride && !y_over_x(prm)) {
       if (EPI == kEpiHeads && prm.v_seq_major) return launch_linear_tiles<T, kEpiHeadsSeqValue>(prm, stream);
       return launch_linear_tiles<T, EPI>(prm, stream);
     }

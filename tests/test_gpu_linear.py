@@ -288,3 +288,29 @@ def test_model_projection_leaves_no_guard_in_a_compiled_caller(gpu_device):
             torch._dynamo.mark_dynamic(value, 0)
             assert torch.equal(call(value), F.linear(value, linear.weight, linear.bias)), rows
     assert counter.frame_count == 1
+
+
+@pytest.mark.parametrize("rows,k", [(1, 256), (300, 256), (300, 64), (20_000, 256)])
+@pytest.mark.parametrize("act", [0, 1])
+def test_256_columns_in_place_through_the_c_abi(gpu_device, rows, k, act):
+    """y over x, 256 columns: the separate buffers' result bit for bit."""
+
+    from solution.kernels.hip import _library
+
+    n, dtype = 256, torch.bfloat16
+    _, (xd, wd, bd) = _operands(rows, k, n, dtype, seed=rows + k, device=gpu_device)
+    padded = torch.zeros(rows, n, dtype=dtype, device=gpu_device)
+    padded[:, :k] = xd
+
+    def call(x, y):
+        status = _library.load_library().sah_linear(
+            x.data_ptr(), wd.data_ptr(), bd.data_ptr(), y.data_ptr(), rows, k, n, n, n, _library.dtype_code(dtype), act,
+            256, 256, 64, 8, 2, _library.stream_handle(gpu_device),
+        )
+        _library.check_status(status, "sah_linear")
+
+    expected = torch.empty_like(padded)
+    call(padded, expected)
+    call(padded, padded)
+    torch.cuda.synchronize()
+    assert torch.equal(padded, expected)
