@@ -11,7 +11,8 @@
 // chosen by size.  The kernel in this file stages its operands through
 // registers and remains for the cases the others do not take: a LayerNorm
 // applied to x on its way into LDS, x rows further apart than the
-// direct loads' 32-bit offsets reach, and y written over x.  It is
+// direct loads' 32-bit offsets reach, y written over x, and up to four K
+// steps of many rows.  It is
 //  * a 256 x 256 output tile per workgroup of 8 wavefronts (2 x 4), each wave
 //    owning 128 rows x 64 columns; K advances 64 at a time through a
 //    double-buffered LDS stage (rows padded by 16 bytes, conflict-free 16-byte
@@ -302,8 +303,12 @@ template <typename T, int EPI, bool LN = false>
 int launch_linear(const LinearParams& prm, hipStream_t stream) {
   if constexpr (!LN) {
     if (prm.x_ld <= kMaxTileStride && !y_over_x(prm)) {
-      if (EPI == kEpiHeads && prm.v_seq_major) return launch_linear_tiles<T, kEpiHeadsSeqValue>(prm, stream);
-      return launch_linear_tiles<T, EPI>(prm, stream);
+      const LinearKernel kernel = linear_kernel_for(prm, EPI);
+      if (kernel != kRegisterStaged) {
+        if (EPI == kEpiHeads && prm.v_seq_major)
+          return launch_linear_tiles<T, kEpiHeadsSeqValue>(prm, kernel, stream);
+        return launch_linear_tiles<T, EPI>(prm, kernel, stream);
+      }
     }
   }
   hipLaunchKernelGGL((linear_kernel<T, EPI, LN>), dim3(prm.num_tiles), dim3(kThreads), 0, stream, prm);

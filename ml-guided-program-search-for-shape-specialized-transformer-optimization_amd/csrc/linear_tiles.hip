@@ -23,6 +23,8 @@
 // spills); loads of the next tile between the epilogue's blocks (1830 us,
 // spills; kept for the 128 x 256 tile, which has the registers).
 
+#include <atomic>
+
 #include "linear_tiles.hpp"
 
 namespace sah {
@@ -316,11 +318,16 @@ __global__ __launch_bounds__(256, 1) void linear_deep_kernel(LinearParams p) {
   }
 }
 
+// The current device's compute units, asked once per device (every Linear call needs them).
 int compute_units() {
-  int device = 0, count = 0;
-  if (hipGetDevice(&device) != hipSuccess ||
-      hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || count <= 0)
+  static std::atomic<int> known[64];
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess || device < 0) return 256;
+  int count = device < 64 ? known[device].load(std::memory_order_relaxed) : 0;
+  if (count > 0) return count;
+  if (hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess || count <= 0)
     return 256;
+  if (device < 64) known[device].store(count, std::memory_order_relaxed);
   return count;
 }
 
@@ -350,15 +357,7 @@ int launch_ring(LinearParams prm, hipStream_t stream) {
 
 }  // namespace
 
-template <typename T, int EPI>
-int launch_linear_tiles(LinearParams prm, hipStream_t stream) {
-  if (prm.seq_len > 1) {
-    // row / seq_len = (row * magic) >> (31 + l), 2^l >= seq_len, for rows below 2^31
-    int l = 1;
-    while ((1ull << l) < (unsigned long long)prm.seq_len) ++l;
-    prm.seq_magic = (uint32_t)((1ull << (31 + l)) / (uint32_t)prm.seq_len + 1);
-    prm.seq_shift = (uint32_t)(l - 1);
-  }
+LinearKernel linear_kernel_for(const LinearParams& prm, int epilogue) {
   // The tile by the rounds that its grid takes on the CUs, each weighed by the
   // time of a round against the 256 x 256 tile's.  Measured (bf16, us, plain
   // Linear / with GELU), 256 x 256, 128 x 256 and the 128 x 128 ring:
@@ -388,19 +387,48 @@ int launch_linear_tiles(LinearParams prm, hipStream_t stream) {
   const double ring128 = rounds(128, 128) * (steps * 0.54 + 2.5);
   const double deep128 = rounds(128, 256) * (steps * 0.66 + 4.0);
   const double deep256 = rounds(256, 256) * (steps * 1.03 + 7.0);
-  if (ring64 <= ring128 && ring64 <= deep128 && ring64 <= deep256) return launch_ring<T, EPI, 64, 64, 4>(prm, stream);
-  if (ring128 <= deep128 && ring128 <= deep256) return launch_ring<T, EPI, 128, 128, 4>(prm, stream);
-  if (deep128 <= deep256) return launch_deep<T, EPI, 128, 256>(prm, stream);
-  return launch_deep<T, EPI, 256, 256>(prm, stream);
+  if (ring64 <= ring128 && ring64 <= deep128 && ring64 <= deep256) return kRing64;
+  if (ring128 <= deep128 && ring128 <= deep256) return kRing128;
+  if (deep128 <= deep256) return kDeep128;
+  // Up to three K steps leave the 256 x 256 tile little but its load latency
+  // and its epilogue, which the register-staged kernel's eight waves pass
+  // faster than four, until (five rounds and more) the chip is busy storing.
+  // Measured (bf16 us, register-staged / 256 x 256; equal bits):
+  //   20002 x 128 -> 512  11.0 / 12.2, GELU 19.3 / 20.9   10000 x 64 -> 1024   9.4 / 10.5
+  //   50000 x 128 -> 512  21.2 / 22.2, GELU 37.6 / 39.5   16384 x 128 -> 1024 13.5 / 13.9
+  //   12000 x 192 -> 768  12.5 / 13.1, GELU 20.8 / 22.0  131072 x 64 -> 1024  76.1 / 67.0
+  // A fourth step only in one round and without GELU, whose arithmetic covers the stores:
+  //   16384 x 256 -> 1024 17.6 / 22.3, GELU 27.0 / 26.3   32768 x 256 -> 512  17.7 / 21.3
+  //   20002 x 256 -> 512  14.6 / 14.5, GELU 22.8 / 23.3   70000 x 256 -> 1024 72.5 / 70.1
+  const int64_t most = prm.k <= 3 * kTileK ? 5 * cus : prm.k == 4 * kTileK && epilogue == kEpiRows ? cus : 0;
+  if (tiles(256, 256) <= most) return kRegisterStaged;
+  return kDeep256;
 }
 
-template int launch_linear_tiles<bf16, kEpiRows>(LinearParams, hipStream_t);
-template int launch_linear_tiles<bf16, kEpiRowsGelu>(LinearParams, hipStream_t);
-template int launch_linear_tiles<bf16, kEpiHeads>(LinearParams, hipStream_t);
-template int launch_linear_tiles<bf16, kEpiHeadsSeqValue>(LinearParams, hipStream_t);
-template int launch_linear_tiles<f16, kEpiRows>(LinearParams, hipStream_t);
-template int launch_linear_tiles<f16, kEpiRowsGelu>(LinearParams, hipStream_t);
-template int launch_linear_tiles<f16, kEpiHeads>(LinearParams, hipStream_t);
-template int launch_linear_tiles<f16, kEpiHeadsSeqValue>(LinearParams, hipStream_t);
+template <typename T, int EPI>
+int launch_linear_tiles(LinearParams prm, LinearKernel kernel, hipStream_t stream) {
+  if (prm.seq_len > 1) {
+    // row / seq_len = (row * magic) >> (31 + l), 2^l >= seq_len, for rows below 2^31
+    int l = 1;
+    while ((1ull << l) < (unsigned long long)prm.seq_len) ++l;
+    prm.seq_magic = (uint32_t)((1ull << (31 + l)) / (uint32_t)prm.seq_len + 1);
+    prm.seq_shift = (uint32_t)(l - 1);
+  }
+  switch (kernel) {
+    case kRing64: return launch_ring<T, EPI, 64, 64, 4>(prm, stream);
+    case kRing128: return launch_ring<T, EPI, 128, 128, 4>(prm, stream);
+    case kDeep128: return launch_deep<T, EPI, 128, 256>(prm, stream);
+    default: return launch_deep<T, EPI, 256, 256>(prm, stream);
+  }
+}
+
+template int launch_linear_tiles<bf16, kEpiRows>(LinearParams, LinearKernel, hipStream_t);
+template int launch_linear_tiles<bf16, kEpiRowsGelu>(LinearParams, LinearKernel, hipStream_t);
+template int launch_linear_tiles<bf16, kEpiHeads>(LinearParams, LinearKernel, hipStream_t);
+template int launch_linear_tiles<bf16, kEpiHeadsSeqValue>(LinearParams, LinearKernel, hipStream_t);
+template int launch_linear_tiles<f16, kEpiRows>(LinearParams, LinearKernel, hipStream_t);
+template int launch_linear_tiles<f16, kEpiRowsGelu>(LinearParams, LinearKernel, hipStream_t);
+template int launch_linear_tiles<f16, kEpiHeads>(LinearParams, LinearKernel, hipStream_t);
+template int launch_linear_tiles<f16, kEpiHeadsSeqValue>(LinearParams, LinearKernel, hipStream_t);
 
 }  // namespace sah

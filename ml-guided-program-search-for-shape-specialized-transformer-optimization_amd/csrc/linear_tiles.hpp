@@ -44,10 +44,15 @@ struct LinearParams {
 // loads reach.
 constexpr int64_t kMaxTileStride = 1 << 22;
 
-// Launch the tile kernel that suits the size on the stream (prm.x_ld <=
-// kMaxTileStride; tiles and grid are set here).
+// The kernel that suits the size (rows, n, k) and epilogue: a tile kernel, or
+// linear_gelu.hip's.
+enum LinearKernel { kRing64, kRing128, kDeep128, kDeep256, kRegisterStaged };
+LinearKernel linear_kernel_for(const LinearParams& prm, int epilogue);
+
+// Launch a tile kernel on the stream (prm.x_ld <= kMaxTileStride; tiles and
+// grid are set here).
 template <typename T, int EPI>
-int launch_linear_tiles(LinearParams prm, hipStream_t stream);
+int launch_linear_tiles(LinearParams prm, LinearKernel kernel, hipStream_t stream);
 
 // The epilogue of the register-staged kernel's TM x TN tile at (m0, n0): bias,
 // activation, one rounding; the tile is staged in smem (TM rows of TN + 8 elements; every wave is past

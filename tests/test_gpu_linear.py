@@ -314,3 +314,24 @@ def test_256_columns_in_place_through_the_c_abi(gpu_device, rows, k, act):
     call(padded, padded)
     torch.cuda.synchronize()
     assert torch.equal(padded, expected)
+
+
+@pytest.mark.parametrize("k", [64, 128, 192, 256])
+@pytest.mark.parametrize("rows,n", [(10_000, 1024), (20_002, 512), (50_000, 256)])
+def test_short_k_of_many_rows(gpu_device, rows, n, k):
+    """About the line to the register-staged kernel (K up to 192, 256 in one round
+    without GELU): rows computed alone (64 x 64 tiles) equal the same rows of the
+    whole call bit for bit, the K order being the same in every kernel."""
+
+    from solution.kernels.ffn import prevalidated_hip_linear, prevalidated_hip_linear_exact_gelu
+
+    for dtype in (torch.bfloat16, torch.float16):
+        _, (xd, wd, bd) = _operands(rows, k, n, dtype, seed=rows + k, device=gpu_device)
+        for call in (prevalidated_hip_linear, prevalidated_hip_linear_exact_gelu):
+            with torch.inference_mode():
+                out, _ = call(xd, wd, bd)
+                parts = [(first, call(xd[first : first + 100].contiguous(), wd, bd)[0])
+                         for first in (0, 256 * 31 - 50, rows - 100)]
+            torch.cuda.synchronize()
+            for first, part in parts:
+                assert torch.equal(out[first : first + 100], part), (dtype, call.__name__, first)
