@@ -258,6 +258,12 @@ int sah_linear_f32(
     int64_t rows, int64_t in_features, int64_t out_features,
     int64_t x_row_stride, int64_t y_row_stride, int activation, sah_stream_t stream);
 
+/* The tile of the kernel that sah_linear takes for these sizes on the current
+ * device (256 compute units where there is none): "64x64", "128x128",
+ * "128x256", "256x256" or "256x256 register-staged"; NULL for sizes it does not
+ * implement.  All give the same bits. */
+const char* sah_linear_kernel(int64_t rows, int64_t in_features, int64_t out_features, int activation);
+
 /* 1 if sah_linear implements this launch, else 0 (mirrors the reference's
  * _launch_config_is_valid, solution/kernels/ffn/triton_linear_exact_gelu.py:29-45). */
 int sah_linear_launch_supported(int block_m, int block_n, int block_k, int num_warps,

@@ -384,6 +384,23 @@ extern "C" int sah_linear(const void* x, const void* weight, const void* bias, v
   return gelu ? launch_linear<f16, kEpiRowsGelu>(prm, s) : launch_linear<f16, kEpiRows>(prm, s);
 }
 
+extern "C" const char* sah_linear_kernel(int64_t rows, int64_t in_features, int64_t out_features, int activation) {
+  if (rows <= 0 || in_features <= 0 || in_features % kBK != 0 || in_features > (1 << 20) || out_features <= 0 ||
+      out_features % kBN != 0 || out_features > (1 << 20))
+    return nullptr;
+  LinearParams prm = {};
+  prm.rows = rows;
+  prm.k = (int)in_features;
+  prm.n = (int)out_features;
+  switch (linear_kernel_for(prm, activation == SAH_ACTIVATION_GELU_EXACT ? kEpiRowsGelu : kEpiRows)) {
+    case kRing64: return "64x64";
+    case kRing128: return "128x128";
+    case kDeep128: return "128x256";
+    case kDeep256: return "256x256";
+    default: return "256x256 register-staged";
+  }
+}
+
 extern "C" int sah_qkv_launch_supported(int block_m, int block_n, int block_k, int num_warps) {
   return block_m == kBM && block_n == kBN && block_k == kBK && num_warps == kWaves;
 }

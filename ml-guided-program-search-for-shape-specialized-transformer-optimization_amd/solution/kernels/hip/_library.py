@@ -81,6 +81,7 @@ _SIGNATURES: dict[str, tuple[list[object], object]] = {
     ),
     "sah_linear": ([_ptr] * 4 + [_i64] * 5 + [_int] * 2 + [_int] * 5 + [_ptr], _int),
     "sah_linear_f32": ([_ptr] * 4 + [_i64] * 5 + [_int, _ptr], _int),
+    "sah_linear_kernel": ([_i64] * 3 + [_int], ctypes.c_char_p),
     "sah_linear_launch_supported": ([_int] * 5, _int),
     "sah_gelu": ([_ptr, _ptr, _i64, _int, _int, _int, _ptr], _int),
     "sah_gelu_launch_supported": ([_int] * 2, _int),

@@ -141,13 +141,14 @@ def test_ineligible_inputs_raise(gpu_device):
 @pytest.mark.parametrize("k", [64, 128, 192, 320])
 @pytest.mark.parametrize(
     "rows,n",
-    # 64 x 64 (twice), 128 x 128, 128 x 256 and 256 x 256 tiles (256 CUs)
+    # 64 x 64 (twice), 128 x 128, 128 x 256 and 256 x 256 tiles (256 CUs; the last
+    # register-staged up to K 192); test_library_abi.py holds the rule to it
     [(1, 256), (129, 512), (777, 4096), (2047, 4096), (8191, 4096)],
 )
 def test_every_tile_kernel_at_its_edges(gpu_device, rows, n, k):
     """Each tile kernel with a partial last row tile and one to five K steps
-    (odd and even: both stages, all prefetch tails; several tiles per
-    workgroup for the largest), with and without GELU, bf16 and fp16, against
+    (odd and even: both stages, all prefetch tails; two tiles per workgroup
+    for the largest), with and without GELU, bf16 and fp16, against
     float64.  The K order is the same in every kernel, so rows computed alone
     (the 64 x 64 tiles) equal the same rows of the whole call bit for bit."""
 
@@ -335,3 +336,17 @@ def test_short_k_of_many_rows(gpu_device, rows, n, k):
             torch.cuda.synchronize()
             for first, part in parts:
                 assert torch.equal(out[first : first + 100], part), (dtype, call.__name__, first)
+
+
+@pytest.mark.parametrize("rows,n,k", [
+    # 128 x 256 tiles, two and three a workgroup: the next tile's loads issued inside
+    # the epilogue, and the counted wait behind its stores (whole and partial last row tiles)
+    (4133, 4096, 64), (4133, 4096, 128), (4133, 4096, 320), (4133, 4096, 1024),
+    (5120, 4096, 64), (5120, 4096, 320),
+    # 256 x 256 tiles, five and six a workgroup, one to four K steps
+    (20_993, 4096, 64), (20_993, 4096, 128), (20_993, 4096, 192), (20_993, 4096, 256),
+])
+def test_persistent_tiles_of_several_rounds(gpu_device, rows, n, k):
+    """The checks of every tile kernel where a workgroup walks several tiles."""
+
+    test_every_tile_kernel_at_its_edges(gpu_device, rows, n, k)

@@ -199,3 +199,32 @@ def test_ineligible_inputs_raise(gpu_device):
         assert can_use_hip_qkv_native_bhsd(x, w, None, num_heads=8)
     # outside inference mode the strict contract refuses (as the reference's does)
     assert not can_use_hip_qkv_native_bhsd(x, w, None, num_heads=8)
+
+
+@pytest.mark.parametrize("batch,seq,layout", [
+    (2, 10_001, "bhsd"),                           # 256 x 256 tiles, four a workgroup
+    (3, 2001, "bhsd"), (3, 2001, "seq_major"),     # 128 x 256 tiles, up to three a workgroup
+    (3, 2000, "bhsd"), (3, 2000, "seq_major"),     # ... with 8-token runs in one sequence
+])
+def test_several_tiles_per_workgroup_match_float64(gpu_device, batch, seq, layout):
+    """Head-major stores of persistent workgroups, every element against float64:
+    one rounding of the result (2^-8) and of 1024 fp32 products and sums."""
+
+    from solution.kernels.projection import hip_qkv_native_bhsd
+
+    d_model, heads = 1024, 16
+    print(f"qkv B{batch} S{seq} {layout}", flush=True)
+    _, (xd, wd, bd) = _operands(batch, seq, d_model, torch.bfloat16, seed=seq, device=gpu_device)
+    with torch.inference_mode():
+        got = hip_qkv_native_bhsd(xd, wd, bd, num_heads=heads, value_layout=layout)[:3]
+    slack = (d_model + 4) * 2.0**-24 * F.linear(xd.double().abs(), wd.double().abs(), bd.double().abs())
+    for name, reference, bound, out in zip(
+        "qkv", _reference(xd, wd, bd, heads), _split_heads(slack, heads), got
+    ):
+        error = (out.double() - reference).abs()
+        assert bool((error <= 2.0**-8 * (reference.abs() + bound) + bound).all()), f"{name}: {float(error.max())}"
+
+
+def _split_heads(packed, heads):
+    batch, seq, width = packed.shape
+    return tuple(p.reshape(batch, seq, heads, -1).transpose(1, 2) for p in packed.split(width // 3, dim=-1))

@@ -340,3 +340,30 @@ def test_python_launch_tables_agree_with_the_library(launch):
                     library.sah_linear_residual_norm_launch_supported(width, rows, warps)
                 )
     assert not linear(256.0, 256, 64, 8, 2) and not qkv(256.0, 256, 64, 8) and not boundary(512.0, 128, 8)
+
+
+_MANY_ROWS = ((10_000, 1024), (20_002, 512), (50_000, 256))
+# Sizes (rows, in, out, activation) of the GPU tests that are there for one kernel
+# of sah_linear, by that kernel: where the rule moves, the tests have to follow.
+LINEAR_KERNEL_CASES = {
+    b"64x64": [(1, 64, 256, 0), (100, 320, 4096, 1), (129, 320, 512, 0), (77, 320, 4096, 0)],
+    b"128x128": [(777, k, 4096, act) for k in (64, 128, 192, 320) for act in (0, 1)],
+    # one tile per workgroup, then two and three, ragged and whole last row tiles
+    b"128x256": [(2047, k, 4096, 0) for k in (64, 128, 192, 320)]
+    + [(rows, k, 4096, act) for rows in (4133, 5120) for k in (64, 128, 320, 1024) for act in (0, 1)]
+    + [(6003, 1024, 3072, 1)],
+    b"256x256": [(8191, 320, 4096, 0), (20_002, 1024, 3072, 1)]
+    + [(20_993, k, 4096, act) for k in (64, 128, 192, 256) for act in (0, 1)],
+    b"256x256 register-staged": [(8191, k, 4096, 0) for k in (64, 128, 192)]
+    + [(rows, k, n, act) for rows, n in _MANY_ROWS for k in (64, 128, 192) for act in (0, 1)]
+    + [(rows, 256, n, 0) for rows, n in _MANY_ROWS],
+}
+
+
+@pytest.mark.parametrize("kernel", sorted(LINEAR_KERNEL_CASES))
+def test_linear_sizes_take_the_kernels_they_are_tests_of(kernel):
+    library = _library.load_library()
+    for case in LINEAR_KERNEL_CASES[kernel]:
+        assert library.sah_linear_kernel(*case) == kernel, case
+    for case in [(0, 64, 256, 0), (1, 32, 256, 0), (1, 64, 128, 0)]:
+        assert library.sah_linear_kernel(*case) is None
