@@ -27,6 +27,7 @@
 // over 64-key LDS tiles, 193 VGPRs):
 //   B4 H8 S777    318 -> 38.7     B2 H12 S1500   807 ->  76
 //   B4 H12 S2500 3031 -> 368      B1 H8 S8192   5956 -> 614 (112 TFLOP/s)
+#include <cfloat>
 #include <cmath>
 
 #include "attention_f32.hpp"
@@ -271,7 +272,9 @@ __global__ __launch_bounds__(kSplit * 64, 2) void attn_fwd_f32_kernel(AttnF32Par
 
 }  // namespace
 
-int launch_attention_f32(const AttnF32Params& p, int batch, hipStream_t stream) {
+int launch_attention_f32(AttnF32Params p, int batch, hipStream_t stream) {
+  // -FLT_MAX where its product with c stays finite, else a little above -FLT_MAX / c
+  p.floor = p.c > 1.0f ? -FLT_MAX / p.c * 0.999999f : -FLT_MAX;
   const int64_t num_q = ceil_div(p.seq_len, kQ);
   const int64_t rows = num_q < 32768 ? num_q : 32768;  // grid y, and z beyond it
   hipLaunchKernelGGL(attn_fwd_f32_kernel,

@@ -19,10 +19,10 @@ struct AttnF32Params {
   int seq_len;
   int heads;
   float c;      // |scale| log2(e), > 0
-  float floor;  // the lowest shift: the most negative float whose product with c is finite
+  float floor;  // set by the launch: the lowest shift, whose product with c is finite
   uint32_t q_and, q_xor;  // the sign of the scale (or a zero scale), on Q
 };
 
-int launch_attention_f32(const AttnF32Params& p, int batch, hipStream_t stream);
+int launch_attention_f32(AttnF32Params p, int batch, hipStream_t stream);
 
 }  // namespace sah

@@ -44,7 +44,6 @@
 //    balances the causal triangle when a head has few query tiles.
 
 #include <algorithm>
-#include <cfloat>
 #include <cmath>
 #include <mutex>
 #include <type_traits>
@@ -917,8 +916,6 @@ int run_attention(
     fp.seq_len = (int)seq_len;
     fp.heads = (int)heads;
     fp.c = prm.c;
-    // -FLT_MAX where its product with c stays finite, else a little above -FLT_MAX / c
-    fp.floor = prm.c > 1.0f ? -FLT_MAX / prm.c * 0.999999f : -FLT_MAX;
     fp.q_and = prm.q_and;
     fp.q_xor = prm.q_xor != 0u ? 0x80000000u : 0u;
     return launch_attention_f32(fp, (int)batch, stream);
