@@ -247,10 +247,10 @@ int sah_linear(
  * nn.Linear and F.gelu of the reference's portable path,
  * solution/transformer.py:291-353).  activation is an enum of sah_linear's
  * (exact GELU through erff).  fp32 accumulation on the fp32 matrix cores, four
- * or eight ranges of K summed in ascending order.  x: [rows, in_features] with row stride x_row_stride;
- * weight: [out_features, in_features] contiguous; bias: [out_features] or
- * NULL; y: [rows, out_features] with row stride y_row_stride, overlapping no
- * input.  in_features a multiple of 128, out_features of 32; row strides
+ * or eight ranges of K summed in ascending order.  x: [rows, in_features] with
+ * row stride x_row_stride; weight: [out_features, in_features] contiguous; bias:
+ * [out_features] or NULL; y: [rows, out_features] with row stride y_row_stride,
+ * overlapping no input.  in_features a multiple of 128, out_features of 32; row strides
  * multiples of 4, tensors 16-byte aligned.
  */
 int sah_linear_f32(

@@ -18,7 +18,8 @@
 // us by library and elementwise kernel, 5.3 here).
 // Measured (us, GPU time, library -> this): 256 x 256 -> 256 63 -> 4.7, 256 x
 // 256 -> 1024 5.6 -> 4.9, 100 x 128 -> 128 11.4 -> 3.8, 256 x 512 -> 256 117
-// -> 5.9, 256 x 1024 -> 256 5.8 -> 6.0; with more tiles than CUs or a longer K
+// -> 5.9, 256 x 1024 -> 256 5.8 -> 6.0, 100 x 640 -> 512 4.9 -> 6.0, 16 x 512 ->
+// 512 4.5 -> 5.8; with more tiles than CUs or a longer K
 // the library is faster (512 x 256 -> 768 5.8 against 7.8, 256 x 2048 -> 256
 // 7.1 against 10.4: the short row segments of the loads).
 #include "sah_common.hpp"

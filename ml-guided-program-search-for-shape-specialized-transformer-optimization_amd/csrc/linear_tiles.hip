@@ -1,22 +1,24 @@
 // Direct-to-LDS tile kernels of the projections (gfx950): Linear, Linear +
 // exact GELU, and the packed QKV projection with its head-major stores.
 //
-// What bounds them: the matrix cores, under the power limit.  The
-// register-staged 8-wave kernel of linear_gelu.hip ran its MFMAs 55% of the
-// time (one __syncthreads per K step with every load behind it, 192 KB of
-// operand reads per step and CU, scalar bias loads in the epilogue) and
-// left most CUs idle for few rows.  Here a 256 x 256 tile is held by four
+// What bounds them: the matrix cores, under the power limit, and the epilogue
+// that nothing covers.  The register-staged 8-wave kernel of linear_gelu.hip
+// waits at one __syncthreads per K step with every load behind it, reads
+// 192 KB of operands per step and CU, loads its bias in scalars in the epilogue,
+// and leaves most CUs idle for few rows.  Here a 256 x 256 tile is held by four
 // waves, one per SIMD, 128 x 128 each: a third fewer LDS reads per MFMA, and
-// one wave's instruction stream keeps its matrix core busy (2180 cycles per
-// K step against 2048 of MFMAs at 20002 x 1024 -> 3072; 72% of all cycles at
-// 65536 x 2048 -> 8192, where the chip then runs at 1.5 GHz).  Measured with
-// the same inputs on one box, before -> after:
+// one wave's instruction stream keeps its matrix core busy: 70% of all cycles
+// at 65536 x 2048 -> 8192, where the chip holds 1.4-1.6 GHz; a tile takes 93 K
+// cycles, 65.5 K of them MFMAs, and 116 K with GELU (counters:
+// profiles/linear_tiles_sq_counters.md).  Measured with the same inputs on one
+// box, before -> after:
 //   65536 x 2048 -> 8192    2567 -> 1710 us (1286 TFLOP/s), GELU 2786 -> 1960 us
 //   20002 x 1024 -> 3072     154 ->  118 us, GELU 179 -> 157 us
 //   777 x 1024 -> 4096        36 ->   13 us, GELU  44 ->  15 us
 //   64 x 4096 -> 1024        102 ->   20 us
-// Few rows take smaller tiles on more CUs: one CU loads about 60 GB/s, and a
-// tile's K steps wait for that.
+// Few rows take smaller tiles on more CUs: one CU loads 50-70 GB/s whatever its
+// tile (first row of the table at linear_kernel_for: (TM + TN) rows of 8 KB each
+// in that time), and a tile's K steps wait for that.
 // Tried and slower at 65536 x 2048 -> 8192: two groups of four waves half a
 // step apart on 128 x 64 wave tiles (1983 us); stores of a tile spread over
 // the next tile's main loop from registers (1790 us: 32-byte segments and
@@ -247,10 +249,11 @@ __global__ __launch_bounds__(256, 1) void linear_ring_kernel(LinearParams p) {
 }
 
 // Persistent workgroups of four waves, one per CU, each walking tiles of its
-// XCD's contiguous run.  A tile's output is finished in registers while the
-// next tile's first loads are under way, and stored between the MFMAs of the
-// next tile's first steps: at the end of a tile all CUs would otherwise wait
-// for 32 MB of stores at once.
+// XCD's contiguous run.  The next tile's first loads are issued before the
+// epilogue (between its blocks on the 128 x 256 tile, which has the registers),
+// and the wait for them counts the epilogue's stores behind them instead of
+// waiting for those too.  The epilogue itself ends before the next tile's
+// products begin.
 template <typename T, int EPI, int TM, int TN>
 __global__ __launch_bounds__(256, 1) void linear_deep_kernel(LinearParams p) {
   typedef GemmTile<T, TM, TN, 2, 2> Tile;
@@ -358,26 +361,24 @@ int launch_ring(LinearParams prm, hipStream_t stream) {
 }  // namespace
 
 LinearKernel linear_kernel_for(const LinearParams& prm, int epilogue) {
-  // The tile by the rounds that its grid takes on the CUs, each weighed by the
-  // time of a round against the 256 x 256 tile's.  Measured (bf16, us, plain
-  // Linear / with GELU), 256 x 256, 128 x 256 and the 128 x 128 ring:
-  //   777 x 1024 -> 4096     24.7 / 33.0    16.6 / 20.7    12.9 / 15.1
-  //   2000 x 1024 -> 4096    26.9 / 35.0    21.9 / 25.8    24.5 / 28.9
-  //   16384 x 2048 -> 512    43.3 / 51.1    35.8 / 40.2    42.3 / 45.8
-  //   16384 x 512 -> 2048    44.2 / 59.2    47.6 / 66.8    57.4 / 71.7
-  //   20002 x 1024 -> 3072    118 / 157      144 / 182      170 / 203
   // The tile by an estimate of its time in us: rounds of its grid on the CUs,
   // each of K / 64 steps and an epilogue.  A step costs what one CU loads
-  // ((TM + TN) rows of 128 bytes at about 60 GB/s) or multiplies; two 64 x 64
-  // workgroups share a CU.  Measured (bf16 Linear, us), 64 x 64, 128 x 128,
+  // ((TM + TN) rows of 128 bytes) or multiplies; two 64 x 64 workgroups share a
+  // CU.  Measured (bf16, us, plain Linear / with GELU), 64 x 64, 128 x 128,
   // 128 x 256 and 256 x 256:
-  //   64 x 4096 -> 1024     19.7   37.4   43.8   68.0
-  //   800 x 2048 -> 512     12.0   20.7   25.1   38.4
-  //   777 x 1024 -> 4096    17.1   13.1   16.5   24.3
-  //   2000 x 1024 -> 3072   24.2   23.7   18.8   25.9
-  //   6000 x 1024 -> 4096   89.1   72.0   57.5   55.6
-  //   16384 x 2048 -> 512            42     36     43
-  //   20002 x 1024 -> 3072          170    144    118
+  //   64 x 4096 -> 1024     19.7         37.4           43.8           68.0
+  //   800 x 2048 -> 512     12.0         20.7           25.1           38.4
+  //   777 x 1024 -> 4096    17.1         12.9 / 15.1    16.6 / 20.7    24.7 / 33.0
+  //   2000 x 1024 -> 3072   24.2         23.7           18.8           25.9
+  //   2000 x 1024 -> 4096                24.5 / 28.9    21.9 / 25.8    26.9 / 35.0
+  //   6000 x 1024 -> 4096   89.1         72.0           57.5           55.6
+  //   16384 x 2048 -> 512                42.3 / 45.8    35.8 / 40.2    43.3 / 51.1
+  //   16384 x 512 -> 2048                57.4 / 71.7    47.6 / 66.8    44.2 / 59.2
+  //   20002 x 1024 -> 3072               170 / 203      144 / 182      118 / 157
+  // The estimates rank the tiles; they are not times: of one clock for all
+  // loads, without GELU, they are up to a third low where the power limit holds
+  // the clock down (20002 x 1024 -> 3072: 94 for 118).  At 6000 x 1024 -> 4096
+  // they take 128 x 256 (43.7 against 47.0) where 256 x 256 is 3% faster.
   const int64_t cus = compute_units();
   const double steps = (double)(prm.k / kTileK);
   auto tiles = [&](int64_t tm, int64_t tn) { return ceil_div(prm.rows, tm) * (prm.n / tn); };

@@ -12,7 +12,8 @@ weight, adds the bias, rounds the update to its fp16 branch dtype, adds it to
 the fp32 residual stream and normalizes, without writing the update.  This
 one (``sah_linear_residual_norm``, csrc/linear_norm.hip) computes the same on a
 bf16 or fp16 stream in two launches (the update passes through an output
-buffer): the update is rounded to the stream dtype, the residual
+buffer), or in one kernel where a short in_features and the row count make it
+faster: the update is rounded to the stream dtype, the residual
 and the normalized rows are the stream dtype (there is no separate fp32
 final-boundary output: the stream is the model dtype), and the projection may
 be rectangular, so it serves both the attention output projection

@@ -28,12 +28,17 @@ from ..hip._library import (
 #   256 x 256 -> 1024   5.6 / 4.9    1024 x 256 -> 1024    8.0 / 13.8
 #   100 x 128 -> 128   11.4 / 3.8
 #   256 x 512 -> 256    117 / 5.9     256 x 2048 -> 256    7.1 / 10.4
-#   256 x 1024 -> 256   5.8 / 6.0
-# A call also costs the host about half of F.linear's (10 us less), which is
-# what bounds a forward of these sizes; with GELU the elementwise launch goes
-# too (256 x 256 -> 1024 8.2 / 5.3).  (The 16-bit tile kernels were tried here
-# too: at 16384 x 512 -> 1536 and 512 -> 512 they are 4-9% faster than the
-# library alone, but the forward of that stack measured the same, 835 us.)
+#   256 x 1024 -> 256   5.8 / 6.0     100 x 640 -> 512     4.9 /  6.0
+#   16 x 512 -> 512     4.5 / 5.8      16 x 1024 -> 4096   5.8 /  6.5
+# Within the rule the library's time is 3.6-172 us, this kernel's 3.1-6.5, at most
+# 1.4 us behind.  A call also costs the host about half of F.linear's (10 us less),
+# which is what bounds a forward of these sizes; with GELU the elementwise launch
+# goes too (256 x 256 -> 1024 8.2 / 5.3).  Replayed from a graph, where the host
+# does not count, whole forwards of four layers gain as well (B1 S16: D 256
+# 223 / 132 us, D 512 231 / 178, D 1024 280 / 190, with the attention's share).
+# (The 16-bit tile kernels were tried here too: at 16384 x 512 -> 1536 and
+# 512 -> 512 they are 4-9% faster than the library alone, but the forward of that
+# stack measured the same, 835 us.)
 _MAX_TILES = 256
 _MAX_IN = 384
 _MAX_IN_SMALL_TILES = 1024
