@@ -93,8 +93,8 @@ def project(module: nn.Linear, value: torch.Tensor, *, gelu: bool = False) -> to
     kernel, or None where it does not serve the call (size, type, layout, or a
     call that something observes)."""
 
-    # first, so that a trace holds no guard on what follows (the sizes)
-    if torch.compiler.is_compiling() or torch.jit.is_tracing():
+    # before the sizes, so that a trace holds no guard on them
+    if value.dtype is not torch.float32 or torch.compiler.is_compiling() or torch.jit.is_tracing():
         return None
     # as registered: reading a parametrized weight computes it (spectral_norm
     # takes a power iteration each time), which is for the module to do once

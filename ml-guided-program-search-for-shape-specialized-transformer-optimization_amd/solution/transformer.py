@@ -281,35 +281,37 @@ class _FP16ShadowLinear(nn.Linear):
         raise AssertionError(f"unhandled projection backend: {backend}")
 
 
-def _is_own_projection(linear: nn.Module) -> bool:
-    return type(linear) is _FP16ShadowLinear and "forward_backend" not in linear.__dict__
+def _takes_small_kernel(linear: nn.Module, backend: ProjectionBackend, plan: ExecutionPlan) -> bool:
+    """Whether a projection may run on the gfx950 kernel of the small fp32
+    projections: an fp32 one of this file's own class (a module put there by the
+    user runs as it is), in the programs on the HIP attention.  Asked of every
+    projection of a forward whose launches are as long on the host as on the
+    GPU, so of registered attributes only."""
 
-
-def _hip_projection(
-    linear: nn.Module, value: torch.Tensor, backend: ProjectionBackend, plan: ExecutionPlan, *, gelu: bool = False
-) -> torch.Tensor | None:
-    """A small fp32 projection, with ``gelu`` the exact GELU of it, on the gfx950
-    kernel: in the programs on the HIP attention, at the sizes where it beats
-    the library GEMM, and only in place of this file's own projection (a module
-    put there by the user runs as it is).  None otherwise."""
-
-    if not plan.uses_hip_attention or backend is not ProjectionBackend.INPUT_DTYPE:
-        return None
-    if not _is_own_projection(linear):
-        return None
-    from .kernels.projection.hip_linear import project
-
-    return project(linear, value, gelu=gelu)
+    return (
+        backend is ProjectionBackend.INPUT_DTYPE
+        and type(linear) is _FP16ShadowLinear
+        and linear._parameters["weight"].dtype is torch.float32
+        and "forward_backend" not in linear.__dict__
+        and plan.uses_hip_attention
+    )
 
 
 def _project(
     linear: nn.Module, value: torch.Tensor, backend: ProjectionBackend, plan: ExecutionPlan
 ) -> torch.Tensor:
-    if backend is ProjectionBackend.INPUT_DTYPE and _is_own_projection(linear):
-        if value.dtype != linear.weight.dtype:  # once, for either path
-            value = value.to(linear.weight.dtype)
-    output = _hip_projection(linear, value, backend, plan)
-    return linear.forward_backend(value, backend) if output is None else output
+    """The projection by ``backend``, a small fp32 one on the gfx950 kernel at the
+    sizes where it beats the library GEMM."""
+
+    if _takes_small_kernel(linear, backend, plan):
+        from .kernels.projection.hip_linear import project
+
+        if value.dtype is not torch.float32:  # once, for either path
+            value = value.to(torch.float32)
+        output = project(linear, value)
+        if output is not None:
+            return output
+    return linear.forward_backend(value, backend)
 
 
 class _SelfAttention(nn.Module):
@@ -568,10 +570,12 @@ class _TransformerBlock(nn.Module):
                 marker, expected_marker=HIP_EXACT_GELU_BACKEND, planned_backend=plan.ffn_backend.value
             )
         else:
-            # a small fp32 projection and its GELU as one launch
-            hidden = _hip_projection(
-                self.ffn_in, normalized, plan.ffn_input_projection_backend, plan, gelu=True
-            )
+            hidden = None
+            if _takes_small_kernel(self.ffn_in, plan.ffn_input_projection_backend, plan):
+                from .kernels.projection.hip_linear import project as hip_project
+
+                # a small fp32 projection and its GELU as one launch
+                hidden = hip_project(self.ffn_in, normalized, gelu=True)
             if hidden is not None:
                 input_compute_dtype = _dtype_name(hidden.dtype)
             else:
