@@ -17,6 +17,8 @@
 // Algorithmic traffic per element: value + update read, residual + normalized
 // written (8 B/element for an all-bf16 boundary).
 
+#include <type_traits>
+
 #include "sah_common.hpp"
 
 namespace sah {
@@ -34,13 +36,17 @@ struct VecIO {
 #pragma unroll
     for (int i = 0; i < N; ++i) out[i] = to_f32(v[i]);
   }
+  template <bool STREAM>
   static __device__ __forceinline__ void store(T* p, const float* in) {
     V v;
 #pragma unroll
     for (int i = 0; i < N; ++i) v[i] = from_f32<T>(in[i]);
     // Streaming store: rows are written once.  Measured on MI355X (bf16,
     // width 1024): 288 -> 277 us for 200000 rows, 27.4 -> 26.5 us for 16384.
-    __builtin_nontemporal_store(v, reinterpret_cast<V*>(p));
+    if (STREAM)
+      __builtin_nontemporal_store(v, reinterpret_cast<V*>(p));
+    else
+      *reinterpret_cast<V*>(p) = v;
   }
 };
 
@@ -63,6 +69,11 @@ __global__ __launch_bounds__(512) void norm_kernel(
     float eps, int rows_per_wave, int rms) {
   constexpr int WIDTH = ITERS * kWave * VEC;
   constexpr int N = ITERS * VEC;
+  // Narrow rows, one a wave, leave through the cache: the projection after them
+  // reads them there.  bf16 B64 S256 D512, four layers: forward 800 us, 830 with
+  // streaming stores (norms 12.2 / 14.6 us, the following projections 29 / 33),
+  // though the norm alone on the same buffers is 14.6 / 11.5.  fp16 rows stream.
+  constexpr bool STREAM = !(ONE_ROW && ITERS == 1 && !std::is_same<TY, f16>::value);
   const int lane = threadIdx.x & (kWave - 1);
   const int wave = threadIdx.x / kWave;
   const int waves = blockDim.x / kWave;
@@ -107,10 +118,12 @@ __global__ __launch_bounds__(512) void norm_kernel(
     if constexpr (HAS_RES) {
 #pragma unroll
       for (int e = 0; e < N; ++e) v[e] = round_to<TX>(v[e] + u[e]);
+      if constexpr (STREAM) {
 #pragma unroll
-      for (int i = 0; i < ITERS; ++i) {
-        const int col = (i * kWave + lane) * VEC;
-        VecIO<TX, VEC>::store(residual + base + col, v + i * VEC);
+        for (int i = 0; i < ITERS; ++i) {
+          const int col = (i * kWave + lane) * VEC;
+          VecIO<TX, VEC>::template store<true>(residual + base + col, v + i * VEC);
+        }
       }
     }
 
@@ -145,10 +158,12 @@ __global__ __launch_bounds__(512) void norm_kernel(
       const float be = has_b ? to_f32(b_raw[e / VEC][e % VEC]) : 0.0f;
       y[e] = fp32_result<TY>((v[e] - mean) * rstd * we + be);
     }
+    if constexpr (HAS_RES && !STREAM)  // one access a lane; beside the other store of its row
+      VecIO<TX, VEC>::template store<false>(residual + base + lane * VEC, v);
 #pragma unroll
     for (int i = 0; i < ITERS; ++i) {
       const int col = (i * kWave + lane) * VEC;
-      VecIO<TY, VEC>::store(normalized + base + col, y + i * VEC);
+      VecIO<TY, VEC>::template store<STREAM>(normalized + base + col, y + i * VEC);
     }
   }
 }
