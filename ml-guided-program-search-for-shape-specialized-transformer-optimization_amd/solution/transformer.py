@@ -288,10 +288,12 @@ def _takes_small_kernel(linear: nn.Module, backend: ProjectionBackend, plan: Exe
     projection of a forward whose launches are as long on the host as on the
     GPU, so of registered attributes only."""
 
+    if backend is not ProjectionBackend.INPUT_DTYPE or type(linear) is not _FP16ShadowLinear:
+        return False
+    weight = linear._parameters.get("weight")  # pruned or normed modules form theirs in a hook
     return (
-        backend is ProjectionBackend.INPUT_DTYPE
-        and type(linear) is _FP16ShadowLinear
-        and linear._parameters["weight"].dtype is torch.float32
+        weight is not None
+        and weight.dtype is torch.float32
         and "forward_backend" not in linear.__dict__
         and plan.uses_hip_attention
     )

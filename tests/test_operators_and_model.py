@@ -233,3 +233,27 @@ def test_projection_converts_its_input_once(hip):
     with torch.no_grad(), Conversions() as mode:
         output = _project(linear, torch.ones(4, 256, dtype=torch.float16), ProjectionBackend.INPUT_DTYPE, plan)
     assert output.dtype == torch.float32 and mode.count == 1
+
+
+@pytest.mark.parametrize("normed", ["pruned", "weight_norm", "spectral_norm"])
+def test_projection_whose_weight_a_hook_forms_runs_as_a_module(normed):
+    """The hook-based utilities of torch.nn.utils keep the module's class and take
+    its registered weight away."""
+
+    from types import SimpleNamespace
+
+    from torch.nn.utils import prune
+
+    from solution.config import ProjectionBackend
+    from solution.transformer import _FP16ShadowLinear, _project
+
+    linear = _FP16ShadowLinear(256, 64)
+    if normed == "pruned":
+        prune.l1_unstructured(linear, "weight", 0.5)
+    else:
+        getattr(torch.nn.utils, normed)(linear)
+    linear.eval()
+    value = torch.randn(4, 256)
+    with torch.no_grad():
+        output = _project(linear, value, ProjectionBackend.INPUT_DTYPE, SimpleNamespace(uses_hip_attention=True))
+        assert torch.equal(output, linear(value))
