@@ -720,10 +720,10 @@ def hip_config(
     attention boundary's norm launch).  ``qkv``
     picks how Q, K and V are produced: VIEW (hipBLASLt packed projection and
     zero-copy views) or HIP_NATIVE_BHSD (the HIP projection writing
-    head-major Q / K and a seq-contiguous V straight from its epilogue).
+    head-major Q, K and V straight from its epilogue).
     ``residual_norm`` picks the boundary: HIP_FUSED (residual + norm after the
     hipBLASLt output projections, with ``norm_launch``) or HIP_LINEAR_FUSED
-    (each output projection fused into its boundary, with ``boundary_launch``,
+    (each output projection and its boundary as one operator, with ``boundary_launch``,
     see hip_linear_boundary_launch).  ``initial_norm`` picks the layer-0
     LayerNorm: HIP (its own kernel, with ``norm_launch``) or HIP_FUSED_QKV
     (fused into the HIP_NATIVE_BHSD projection, which it requires)."""
