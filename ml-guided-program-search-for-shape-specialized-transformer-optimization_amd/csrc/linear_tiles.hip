@@ -169,8 +169,11 @@ __device__ __forceinline__ void store_wave(const LinearParams& p, unsigned char*
           run[t] = *reinterpret_cast<const T*>(area + (row0 + t) * (CPR * 16) + slot(row0 + t, vcol >> 3) * 16 + (vcol & 7) * 2);
         uint32_t b, s;
         seq_div(p, (uint32_t)m, b, s);
-        if (p.seq_aligned && m + 8 <= p.rows) {
-          store16(dst + (((int64_t)b * p.heads + vh) * p.head_dim + ve) * p.v_ld + s, __builtin_bit_cast(u32x4, run));
+        if (m + 8 <= p.rows && s + 8 <= (uint32_t)p.seq_len) {
+          // 16-byte aligned only where seq_len % 8 == 0; the copy is one 16-byte store all the
+          // same, which takes any element's address (B3 S5001 D768 167 -> 92 us against
+          // element stores, register-staged 134; D1024 167 -> 103)
+          __builtin_memcpy(dst + (((int64_t)b * p.heads + vh) * p.head_dim + ve) * p.v_ld + s, &run, 16);
         } else {
 #pragma unroll
           for (int t = 0; t < 8; ++t) {

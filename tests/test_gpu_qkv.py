@@ -201,19 +201,21 @@ def test_ineligible_inputs_raise(gpu_device):
     assert not can_use_hip_qkv_native_bhsd(x, w, None, num_heads=8)
 
 
-@pytest.mark.parametrize("batch,seq,layout", [
-    (2, 10_001, "bhsd"),                           # 256 x 256 tiles, four a workgroup
-    (3, 2001, "bhsd"), (3, 2001, "seq_major"),     # 128 x 256 tiles, up to three a workgroup
-    (3, 2000, "bhsd"), (3, 2000, "seq_major"),     # ... with 8-token runs in one sequence
+@pytest.mark.parametrize("batch,seq,d_model,layout", [
+    (2, 10_001, 1024, "bhsd"),                                 # 256 x 256 tiles, four a workgroup
+    (3, 2001, 1024, "bhsd"), (3, 2001, 1024, "seq_major"),     # 128 x 256 tiles, up to three a workgroup
+    (3, 2000, 1024, "bhsd"), (3, 2000, 1024, "seq_major"),     # ... with 8-token runs in one sequence
+    (3, 5001, 768, "seq_major"),                               # 256 x 256, runs at every offset
+    (1201, 5, 256, "seq_major"), (600, 9, 512, "seq_major"),   # every run, or seven of eight, over a boundary
 ])
-def test_several_tiles_per_workgroup_match_float64(gpu_device, batch, seq, layout):
+def test_several_tiles_per_workgroup_match_float64(gpu_device, batch, seq, d_model, layout):
     """Head-major stores of persistent workgroups, every element against float64:
-    one rounding of the result (2^-8) and of 1024 fp32 products and sums."""
+    one rounding of the result (2^-8) and of d_model fp32 products and sums."""
 
     from solution.kernels.projection import hip_qkv_native_bhsd
 
-    d_model, heads = 1024, 16
-    print(f"qkv B{batch} S{seq} {layout}", flush=True)
+    heads = d_model // 64
+    print(f"qkv B{batch} S{seq} D{d_model} {layout}", flush=True)
     _, (xd, wd, bd) = _operands(batch, seq, d_model, torch.bfloat16, seed=seq, device=gpu_device)
     with torch.inference_mode():
         got = hip_qkv_native_bhsd(xd, wd, bd, num_heads=heads, value_layout=layout)[:3]
