@@ -12,7 +12,7 @@
 // registers and remains for the cases the others do not take: a LayerNorm
 // applied to x on its way into LDS, x rows further apart than the
 // direct loads' 32-bit offsets reach, y written over x, and up to four K
-// steps of many rows.  It is
+// steps of many rows (linear_kernel_for).  It is
 //  * a 256 x 256 output tile per workgroup of 8 wavefronts (2 x 4), each wave
 //    owning 128 rows x 64 columns; K advances 64 at a time through a
 //    double-buffered LDS stage (rows padded by 16 bytes, conflict-free 16-byte

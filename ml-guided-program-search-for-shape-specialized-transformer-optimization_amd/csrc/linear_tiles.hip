@@ -404,7 +404,20 @@ LinearKernel linear_kernel_for(const LinearParams& prm, int epilogue) {
   // A fourth step only in one round and without GELU, whose arithmetic covers the stores:
   //   16384 x 256 -> 1024 17.6 / 22.3, GELU 27.0 / 26.3   32768 x 256 -> 512  17.7 / 21.3
   //   20002 x 256 -> 512  14.6 / 14.5, GELU 22.8 / 23.3   70000 x 256 -> 1024 72.5 / 70.1
-  const int64_t most = prm.k <= 3 * kTileK ? 5 * cus : prm.k == 4 * kTileK && epilogue == kEpiRows ? cus : 0;
+  // Head-major (K is 256 or more there) always, but a seq-contiguous value only up to six rounds
+  // and where its 8-token runs are aligned, as that kernel wants them (us at D 256, register-staged /
+  // 256 x 256, then with such a value):
+  //   B2 S8192   15.7 / 16.9, 18.9 / 22.9   B16 S4096  48.2 / 51.9, 52.8 / 49.7
+  //   B1 S12000  15.3 / 16.3, 17.8 / 22.5   B20 S4000  58.2 / 65.8, 60.7 / 68.3
+  //   B3 S5001   15.9 / 16.8, 51.3 / 23.3   B64 S1600  73.0 / 83.0, 76.1 / 83.0
+  //                                         B1 S300000  233 / 243,   252 / 233
+  int64_t most = 0;
+  if (prm.k <= 3 * kTileK)
+    most = 5 * cus;
+  else if (prm.k == 4 * kTileK && epilogue == kEpiRows)
+    most = cus;
+  else if (prm.k == 4 * kTileK && epilogue == kEpiHeads)
+    most = !prm.v_seq_major ? INT64_MAX : prm.seq_aligned ? 6 * cus : 0;
   if (tiles(256, 256) <= most) return kRegisterStaged;
   return kDeep256;
 }

@@ -206,6 +206,8 @@ def test_ineligible_inputs_raise(gpu_device):
     (3, 2001, 1024, "bhsd"), (3, 2001, 1024, "seq_major"),     # 128 x 256 tiles, up to three a workgroup
     (3, 2000, 1024, "bhsd"), (3, 2000, 1024, "seq_major"),     # ... with 8-token runs in one sequence
     (3, 5001, 768, "seq_major"),                               # 256 x 256, runs at every offset
+    (1, 12_000, 256, "bhsd"), (1, 12_000, 256, "seq_major"),   # register-staged
+    (3, 5001, 256, "bhsd"), (10, 4001, 256, "bhsd"), (3, 5001, 256, "seq_major"),
     (1201, 5, 256, "seq_major"), (600, 9, 512, "seq_major"),   # every run, or seven of eight, over a boundary
 ])
 def test_several_tiles_per_workgroup_match_float64(gpu_device, batch, seq, d_model, layout):
